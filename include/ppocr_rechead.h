@@ -41,7 +41,7 @@ extern "C" {
 /* How the projection's inner products are computed.  All modes accumulate in fp32 and
  * apply the per-class scale and bias in fp32 in the epilogue. */
 typedef enum {
-    PPOCR_MODE_FP32_FMA = 0, /* fp32 vector FMA over dequantised weights */
+    PPOCR_MODE_FP32_FMA = 0, /* fp32 products and sums over dequantised weights */
     PPOCR_MODE_BF16X1 = 1,   /* bf16 MFMA, activation rounded to 1 bf16 term */
     PPOCR_MODE_BF16X2 = 2,   /* bf16 MFMA, activation split into 2 bf16 terms */
     PPOCR_MODE_BF16X3 = 3,   /* bf16 MFMA, activation split into 3 bf16 terms; for an

@@ -551,12 +551,19 @@ int mode_cfg(const ppocr_rh* h, int mode, int* cfg) {
     return PPOCR_OK;
 }
 
+// Vocabulary chunks of the fp32 statistics pass: the count with the fewest tile times, its
+// grid running in rounds of 512 workgroups (2 per CU) and a workgroup costing about one tile
+// beside its own; at most as many as make 1024 workgroups.
 int fma_nsplit(int64_t m, int64_t n) {
-    const int64_t mblocks = (m + kFmaRowsPerBlock - 1) / kFmaRowsPerBlock;
+    const int64_t mblocks = std::max<int64_t>((m + kFmaRowsPerBlock - 1) / kFmaRowsPerBlock, 1);
     const int64_t ntiles = (n + kFmaCols - 1) / kFmaCols;
-    int64_t ns = (1024 + mblocks - 1) / std::max<int64_t>(mblocks, 1);
-    ns = std::min<int64_t>(std::max<int64_t>(ns, 1), std::min<int64_t>(ntiles, 1024));
-    return (int)ns;
+    const int64_t top = std::max<int64_t>(std::min<int64_t>((1024 + mblocks - 1) / mblocks, std::min<int64_t>(ntiles, 1024)), 1);
+    int64_t best = 1, best_cost = INT64_MAX;
+    for (int64_t ns = 1; ns <= top; ++ns) {
+        const int64_t cost = (mblocks * ns + 511) / 512 * ((ntiles + ns - 1) / ns + 1);
+        if (cost < best_cost) best = ns, best_cost = cost;
+    }
+    return (int)best;
 }
 
 int nsplit_for(const ppocr_rh* h, int64_t m, int cfg) {

@@ -186,7 +186,7 @@ int launch_probs_mfma(int cfg, const TileGeom& tg, const uint8_t* rec, const uin
 // Epilogues of the projection kernels: logits, probabilities, per-chunk softmax statistics.
 enum Epi : int { EPI_LOGITS = 0, EPI_PROBS = 1, EPI_STATS = 2 };
 
-// fp32 vector FMA path over the packed int8 weights (q != null) or fp32 weights (w != null).
+// fp32 path (products and sums in fp32) over the packed int8 weights (q != null) or fp32 weights (w != null).
 int launch_logits_fma(const int8_t* q, const float* w, const float* scale, const float* bias,
                       const float* a, int64_t m, int64_t n, int64_t k, float* out, hipStream_t st);
 constexpr int kFmaRowsPerBlock = 128, kFmaCols = 128;  // rows and classes of a workgroup's tile
