@@ -1319,7 +1319,8 @@ int neck_f16_exponent(double bound) {
     return e;
 }
 
-bool neck_f16_bounds_ok(const NeckHost& nh, int (*exps)[7]) {
+constexpr int kNeckExps = 10;
+bool neck_f16_bounds_ok(const NeckHost& nh, int (*exps)[kNeckExps]) {
     const int64_t D = nh.dim, H = nh.hidden;
     constexpr double kLimit = 16384.0;  // a quarter of fp16's largest finite value
     auto amax = [](const float* v, int64_t n) {
@@ -1359,6 +1360,9 @@ bool neck_f16_bounds_ok(const NeckHost& nh, int (*exps)[7]) {
         exps[i][4] = neck_f16_exponent(amax(b.fc2_w, H * D));              // fc2's weights
         exps[i][5] = neck_f16_exponent(y2);                                // LN2's output
         exps[i][6] = neck_f16_exponent(hs);                                // the hidden layer
+        exps[i][7] = neck_f16_exponent(amax(b.qkv_w, D * 3 * D));          // qkv's weights
+        exps[i][8] = neck_f16_exponent(y1);                                // LN1's output
+        exps[i][9] = neck_f16_exponent(amax(b.proj_w, D * D));             // proj's weights
     }
     return true;
 }
@@ -1392,7 +1396,7 @@ int neck_create(const NeckHost& nh, int device, ppocr_rn_t** out) {
     parts.push_back({nh.lnf_w, D});
     parts.push_back({nh.lnf_b, D});
     // the fp16 planes of each block's four weights, as float-sized parts after the rest
-    int exps[kNeckMaxBlocks][7] = {};
+    int exps[kNeckMaxBlocks][kNeckExps] = {};
     const bool f16 = neck_f16_bounds_ok(nh, exps);
     std::vector<std::vector<uint16_t>> planes;
     std::vector<std::vector<float>> padded_bias;
@@ -1417,6 +1421,9 @@ int neck_create(const NeckHost& nh, int device, ppocr_rn_t** out) {
             padded_bias.push_back(std::move(bp));
         }
         for (const auto& bp : padded_bias) parts.push_back({bp.data(), (int64_t)bp.size()});
+        // the block kernels' planes, built on the device (no host data)
+        for (size_t i = 0; i < nh.blocks.size(); ++i)
+            for (int halves : kNeckFragHalves) parts.push_back({nullptr, halves / 2});
     }
     int64_t total = 0;
     for (const auto& pt : parts) total += (pt.second + 3) / 4 * 4;  // each part 16-byte aligned
@@ -1435,13 +1442,13 @@ int neck_create(const NeckHost& nh, int device, ppocr_rn_t** out) {
     h->device_bytes = (size_t)total * 4;
     std::vector<float> host((size_t)total, 0.0f);
     std::vector<const float*> dev_ptr;
-    int64_t off = 0;
+    int64_t off = 0, uploaded = 0;  // the parts without host data come last
     for (const auto& pt : parts) {
-        std::memcpy(host.data() + off, pt.first, (size_t)pt.second * 4);
+        if (pt.first) std::memcpy(host.data() + off, pt.first, (size_t)pt.second * 4), uploaded = off + pt.second;
         dev_ptr.push_back(h->d_weights + off);
         off += (pt.second + 3) / 4 * 4;
     }
-    PPOCR_HIP(hipMemcpy(h->d_weights, host.data(), (size_t)total * 4, hipMemcpyHostToDevice));
+    PPOCR_HIP(hipMemcpy(h->d_weights, host.data(), (size_t)uploaded * 4, hipMemcpyHostToDevice));
     NeckDev& nd = h->dev;
     nd.dim = (int)D;
     nd.heads = (int)nh.heads;
@@ -1482,8 +1489,17 @@ int neck_create(const NeckHost& nh, int device, ppocr_rn_t** out) {
         b.mlp_e2 = exps[i][4];
         b.mlp_ey = exps[i][5];
         b.mlp_eh = exps[i][6];
+        b.qkv_e = exps[i][7];
+        b.qkv_ey = exps[i][8];
+        b.proj_e = exps[i][9];
     }
     for (size_t i = 0; f16 && i < nh.blocks.size(); ++i) nd.block[i].qkv_bp = dev_ptr[q++];
+    for (size_t i = 0; f16 && i < nh.blocks.size(); ++i) {
+        NeckBlockDev& b = nd.block[i];
+        for (const uint16_t** f : {&b.qkv_f, &b.proj_f, &b.fc1_f, &b.fc2_f}) *f = reinterpret_cast<const uint16_t*>(dev_ptr[q++]);
+        if (int e = launch_neck_fragments(b, nullptr)) return e;
+    }
+    if (f16) PPOCR_HIP(hipStreamSynchronize(nullptr));
     *out = h.release();
     return PPOCR_OK;
 }

@@ -8,7 +8,8 @@
 // and Mul for the swish, and the residual Adds.
 //
 // gfx950 layout: the token rows of all lines packed back to back, channels contiguous
-// ([m][D], D = 120).  Four kinds of kernels:
+// ([m][D], D = 120).  Batches of up to kNeckFusedRows rows on fp16 halves take the block kernels of
+// neck_fused.hip.  Here, four kinds of kernels:
 //   neck_gemm16_kernel rows x W[K][N] on fp16 halves of both operands (three exact products
 //                      per f16 MFMA step, fp32 sums), with the LayerNorm of the rows folded
 //                      into the operand load and bias, swish and the residual Add folded into
@@ -1302,16 +1303,17 @@ int gemm_go(const float* a, int64_t m, const float* w, int n, const float* bias,
 
 }  // namespace
 
+int NeckMark::operator()(const char* name) const {
+    if (!marks) return PPOCR_OK;
+    if (marks->count >= marks->capacity) return fail(PPOCR_ERR_INVALID_ARG, "RecNeckHip: too few events");
+    PPOCR_HIP(hipEventRecord(marks->events[marks->count], st));
+    marks->names[marks->count++] = name;
+    return PPOCR_OK;
+}
+
 int launch_neck(const NeckDev& nk, const float* x_in, const float* shortcut_in, int64_t m, const int64_t* line_off,
                 int64_t lines, int64_t line_len, int layout, float* out, float* ws, hipStream_t st, NeckMarks* marks) {
-    // an event after the kernel just launched (and its name), when marks are asked for
-    auto mark = [&](const char* name) -> int {
-        if (!marks) return PPOCR_OK;
-        if (marks->count >= marks->capacity) return fail(PPOCR_ERR_INVALID_ARG, "RecNeckHip: too few events");
-        PPOCR_HIP(hipEventRecord(marks->events[marks->count], st));
-        marks->names[marks->count++] = name;
-        return PPOCR_OK;
-    };
+    const NeckMark mark{marks, st};
     const int D = nk.dim, H = nk.hidden;
     if (D != kNeckDim || H != kNeckHidden || nk.heads * kNeckHeadDim != D)
         return fail(PPOCR_ERR_INVALID_ARG, "RecNeckHip: unsupported neck geometry");
@@ -1321,6 +1323,12 @@ int launch_neck(const NeckDev& nk, const float* x_in, const float* shortcut_in, 
     if (lines <= 0 || (!line_off && line_len <= 0)) return fail(PPOCR_ERR_INVALID_ARG, "RecNeckHip: no lines");
     if (lines > 0x7fffffffLL) return fail(PPOCR_ERR_INVALID_ARG, "RecNeckHip: too many lines");
     if (int e = mark("start")) return e;
+    // up to a workgroup per CU the block kernels are faster (one line 93 -> 33 us, 16384 rows
+    // 100 -> 76); past that their second round is not (32768 rows: 145 against 141, 17000: 145
+    // against 101)
+    if (nk.f16 && m <= kNeckFusedRows)
+        return launch_neck_fused(nk, x_in, shortcut_in, m, line_off, lines, line_len,
+                                 layout == PPOCR_NECK_CHANNELS_FIRST, out, ws, st, mark);
     float* x = ws;                       // residual stream [m][D]
     float* sc = x + m * D;               // shortcut rows [m][D]
     float* qkv = sc + m * D;             // [m][3D], or [m][kNeckQkvPad] on fp16 halves

@@ -34,6 +34,12 @@ struct NeckBlockDev {
     // of 8][unit] then fc2's planes of the matching contraction block as [plane][chunk]
     // [output column (128)], 8 halves per entry, zeros past the hidden units and columns
     const uint16_t* mlp_h;
+    // the planes of qkv, proj, fc1 and fc2 for the block kernels of small batches
+    // (neck_fused.hip), each weight times 2^e before the split, in the order of the MFMA operand
+    // registers: per tile of 16 output columns and step of 32 contraction values
+    // [plane][lane][8], lane (c, g) column c at contraction values 8 g .. 8 g + 7; zeros past
+    // the columns and the contraction (qkv's columns and proj's contraction padded per head)
+    const uint16_t *qkv_f, *proj_f, *fc1_f, *fc2_f;
     // the attention's operands scaled by powers of two before the fp16 split (q * scale by
     // 2^attn_eq, k by 2^attn_ek, v by 2^attn_ev), chosen from their bounds so that the halves
     // of all but negligible values stay above fp16's subnormals
@@ -42,6 +48,9 @@ struct NeckBlockDev {
     // weights times 2^mlp_e1 and 2^mlp_e2, the kernel scales LN2's output by 2^mlp_ey and
     // the hidden layer by 2^mlp_eh before their splits, and each product by the inverse
     int mlp_e1, mlp_e2, mlp_ey, mlp_eh;
+    // the block kernels' other scalings: qkv's and proj's weights, LN1's output (the
+    // attention's output is scaled by 2^attn_ev)
+    int qkv_e, proj_e, qkv_ey;
 };
 
 struct NeckDev {
@@ -80,8 +89,24 @@ struct NeckMarks {
     int capacity;
     int count;
 };
+// Records the event that ends a kernel of the forward, when marks are asked for.
+struct NeckMark {
+    NeckMarks* marks;
+    hipStream_t st;
+    int operator()(const char* name) const;
+};
 int launch_neck(const NeckDev& nk, const float* x_in, const float* shortcut_in, int64_t m, const int64_t* line_off,
                 int64_t lines, int64_t line_len, int layout, float* out, float* ws, hipStream_t st,
                 NeckMarks* marks = nullptr);
+// The same on fp16 halves (nk.f16) in one launch per block and one before the first, for at most
+// kNeckFusedRows rows (arguments checked by launch_neck); cf: channels-first input and shortcut.
+// Fills qkv_f .. fc2_f of a block (kNeckFragHalves in all, in that order) from its uploaded
+// weights and exponents.
+constexpr int kNeckFragHalves[4] = {24 * 4 * 1024, 8 * 4 * 1024, 16 * 4 * 1024, 8 * 8 * 1024};
+int launch_neck_fragments(const NeckBlockDev& k, hipStream_t st);
+constexpr int64_t kNeckFusedRows = 64 * 256;
+int launch_neck_fused(const NeckDev& nk, const float* x_in, const float* shortcut, int64_t m, const int64_t* line_off,
+                      int64_t lines, int64_t line_len, bool cf, float* out, float* ws, hipStream_t st,
+                      const NeckMark& mark);
 
 }  // namespace ppocr

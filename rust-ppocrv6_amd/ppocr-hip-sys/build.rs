@@ -21,6 +21,7 @@ const SOURCES: &[&str] = &[
     "head_fma.hip",
     "softmax_ctc.hip",
     "neck.hip",
+    "neck_fused.hip",
     "safetensors.cpp",
     "model_graph.cpp",
 ];
@@ -41,6 +42,8 @@ const FLAGS: &[&str] = &[
 // accumulator-register copies before their vector work).
 fn file_flags(src: &str) -> &'static [&'static str] {
     if src == "neck.hip" {
+        &["-mllvm", "-amdgpu-mfma-vgpr-form=1"]
+    } else if src == "neck_fused.hip" {
         &["-mllvm", "-amdgpu-mfma-vgpr-form=1"]
     } else {
         &[]
