@@ -259,15 +259,30 @@ static int vec_ok(const float* a, int64_t k) {
     return ((reinterpret_cast<uintptr_t>(a) & 15) == 0 && (k & 3) == 0) ? 1 : 0;
 }
 
-// Vocabulary chunks of the writer (128-row workgroups, one per CU).  HBM write bandwidth
-// falls with the number of row segments written at once (measured on the logits layout,
-// 30720 x 18710 fp32: 4.3 TB/s with one chunk per row, 3.0 with two, 2.6 with eight), so a
-// batch with enough rows to fill the GPU walks each row's vocabulary in one pass; small
-// batches split the vocabulary to fill it.
+// Vocabulary chunks of the writer (128-row workgroups, one per CU, so 32 per XCD at once).  The
+// count whose grid fills one round best: a multiple of 8 (every XCD its own chunks of every row
+// block) or 4, 2, 1 (an XCD takes one chunk of every 2nd, 4th, 8th row block).  Where that
+// leaves an XCD barely over half full, several rounds of smaller chunks are faster (logits of
+// the 18710-class head, us): 18 row blocks 54 in 8 chunks, 44 in 24; 33 blocks 104 in 4, 95 in
+// 24; fuller ones are not: 23 blocks 55 in 8, 64 in 24; 47 blocks 124 in 4, 144; 94 blocks 244 in
+// 2, 265 in 8; 130 blocks 362 in 1, 372 in 8; 240 blocks 643 in 1, 649 in 8.  (Doubling the count
+// until 192 workgroups, as before, put 18 blocks in 16 chunks: 288 workgroups, two rounds, 60
+// us; 33 in 8: 120; 94 in 4: 283; 130 in 2: 492, its second round 4 workgroups.)
+constexpr int kMaxWriterChunks = 128;
 static int rows_nsplit(int64_t mblocks) {
-    int ns = 1;
-    while (mblocks * ns < 192 && ns < 64) ns *= 2;
-    return ns;
+    constexpr int64_t kSlots = 32;  // workgroups of an XCD at once
+    if (mblocks <= kSlots) {
+        const int64_t ns = std::min<int64_t>(8 * (kSlots / mblocks), kMaxWriterChunks);
+        // up to 21 row blocks, two rounds of 24 chunks
+        return ns == 8 && 3 * mblocks <= 2 * kSlots ? 24 : (int)ns;
+    }
+    if (mblocks > 8 * kSlots) {  // more than a round in one chunk: 8 unless its last round is well filled
+        const int64_t last = (mblocks + 7) / 8 % kSlots;
+        return last == 0 || last > 18 ? 1 : 8;
+    }
+    int ns = 4;
+    while (ns > 1 && (mblocks * ns + 7) / 8 > kSlots) ns /= 2;
+    return ns > 1 && (mblocks * ns + 7) / 8 <= 18 ? 24 : ns;
 }
 
 // Row-block slots of a rescue pass: its grid is sized before the number of guarded rows
@@ -326,7 +341,7 @@ static int launch_rows(int cfg, int epi, const TileGeom& tg, const uint8_t* rec,
     const GuardLimits limit = !guarded ? none
                               : epi == 1 ? stats_limit_of(cfg, *guard)
                                          : GuardLimits{guard->amax_limit, INFINITY, INFINITY};
-    if (guarded) {
+    if (guarded && !guard->emptied) {
         // a replay of this call (same epoch) must start from an empty list too
         guard_reset_kernel<<<1, 1, 0, st>>>(guard->header, guard->epoch);
         PPOCR_HIP(hipGetLastError());

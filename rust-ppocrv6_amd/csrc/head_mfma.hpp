@@ -980,6 +980,8 @@ constexpr int writer_ring() {
 // class of 16 rows, so each store instruction writes 32 consecutive classes of two rows.
 // GATHER: the rows are the entries of the guard list (the rescue of guarded rows); a
 // workgroup then takes several row blocks and the producer streams the tiles once per block.
+// Most classes whose 32-row blocks are addressed by 32-bit offsets.
+constexpr int kBufferClasses = 1 << 24;
 template <int C, int G, int EPI, bool GATHER>
 __global__ __launch_bounds__(64 * (kWriterWaves + 1), 1) void rows_w_kernel(
     const float* __restrict__ a, int64_t m, int k, int vec, const uint8_t* __restrict__ rec, int tiles, int n,
@@ -1009,7 +1011,11 @@ __global__ __launch_bounds__(64 * (kWriterWaves + 1), 1) void rows_w_kernel(
     // with the write stream running, L2 read latency rose from about 300 cycles (one tile
     // re-read) to 1450 and write latency from 320 to 1000 (TCP_TCC_*_REQ_LATENCY), and the
     // logits kernel took 843 us instead of 648 (dense batch, same box).
-    const int rot = (int)(((int64_t)mbi * 149) % ntiles);
+    // The starts of an XCD's workgroups (ids 8 apart) follow the golden ratio (8 x 5063 / 2^16 =
+    // 0.618), spread over the chunk whatever its length; the XCDs' own start an eighth of that
+    // apart.  (149 tiles per row block, as before, put the starts of chunks of 37, 74 or 147 tiles
+    // one or two tiles apart: 30720 rows in 4 chunks 779 us, 649 so.)
+    const int rot = (int)(((int64_t)((blockIdx.x * 5063u) & 0xffffu) * ntiles) >> 16);
     const int64_t total = nblk * ntiles;
 
     const int tid = threadIdx.x, lane = tid & 63, i = lane & 31, h = lane >> 5;
@@ -1086,6 +1092,12 @@ __global__ __launch_bounds__(64 * (kWriterWaves + 1), 1) void rows_w_kernel(
             }
         }
 
+        // the wave's 32 rows of the output, as far as the batch goes (a raw buffer: stores at or past
+        // its end are dropped)
+        const int64_t brows = GATHER || n > kBufferClasses ? 0 : min(max(m - j0, (int64_t)0), (int64_t)32);
+        const auto obuf = __builtin_amdgcn_make_buffer_rsrc(out + (brows > 0 ? j0 : 0) * n, 0,
+                                                            (unsigned)(brows * n * 4), 0x00020000);
+
         for (int t = t0; t < t1; ++t) {
             const uint8_t* buf = lds + cslot * GE::BUF;
             cslot = cslot + 1 == R ? 0 : cslot + 1;
@@ -1126,7 +1138,18 @@ __global__ __launch_bounds__(64 * (kWriterWaves + 1), 1) void rows_w_kernel(
                     v[r] = __builtin_amdgcn_exp2f(fmaf(acc[r], c0, c1) - rmax[r]) * rinv[r];
                 }
             }
-            if (all_valid && tt * 32 + 32 <= n) {
+            if (!GATHER && n <= kBufferClasses) {
+                // one 32-bit offset per row from the wave's first row; the buffer ends with the
+                // batch, so rows past it are dropped by the bounds check, and so are classes past
+                // n, moved past any end.  A branch per row instead made the compiler wait for the
+                // stores in flight: a batch that is no multiple of 128 rows waited for its last
+                // row block (12000 rows in one chunk: 94 row blocks 381 us, whole ones 326).
+                const unsigned o = col < n ? ((unsigned)(4 * h) * (unsigned)n + (unsigned)col) * 4u : 0xFFFFFFFFu;
+                const unsigned add = col < n ? 4u * (unsigned)n : 0u;
+#pragma unroll
+                for (int r = 0; r < 16; ++r)
+                    __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v[r]), obuf, o + (8 * (r >> 2) + (r & 3)) * add, 0, 0);
+            } else if (all_valid && tt * 32 + 32 <= n) {
 #pragma unroll
                 for (int r = 0; r < 16; ++r) out[(int64_t)orow[r] * n + col] = v[r];
             } else if (col < n) {

@@ -119,6 +119,9 @@ struct Guard {
     bool stats_noref;
     const FmaWeights& fma;  // the head's fp32 weights, for a rescue in fp32 FMA
     uint8_t* skip;          // a byte per 128 rows: the statistics pass's skipped row blocks
+    // the list was emptied earlier in this call under the same epoch (by the statistics
+    // merge before a probabilities pass): no reset launch
+    bool emptied = false;
 };
 
 // Supported group counts (k = 113..120 and k = 73..80, the PP-OCRv6 small and tiny heads).
