@@ -102,18 +102,26 @@ struct DeviceGuard {
 // inputs, outputs and workspace out in it, and gives it back, so a call costs its copies
 // and kernels rather than allocations.  Inputs and outputs of up to kStageBytes move as
 // one copy each way through the pinned buffer; larger ones are copied directly.  Calls
-// running at the same time take different arenas.  Arenas above kArenaKeepBytes are freed
+// running at the same time take different arenas.  The staged inputs go to the device in pieces,
+// by a kernel that reads the pinned buffer, so a piece crosses PCIe while the next one is being
+// copied into the buffer and the call's kernels follow on the same queue; decoded results of
+// up to kDirectBytes are written by the kernels into the pinned buffer themselves.  (An A4 page,
+// 2245 rows from host arrays: 107 us with one asynchronous copy each way, 96 so.)
+// Arenas above kArenaKeepBytes are freed
 // after the call instead of kept (the logits of a large batch need gigabytes once).  The
 // pool lives until the process ends.
 constexpr size_t kArenaKeepBytes = 256u << 20;
 constexpr size_t kStageBytes = 4u << 20;
+constexpr size_t kDirectBytes = 256u << 10;  // after the stage, in the same pinned buffer
+constexpr size_t kStagePiece = 512u << 10;
 
 struct HostArena {
     int device = -1;
     hipStream_t stream = nullptr;
     uint8_t* base = nullptr;
     size_t cap = 0;
-    uint8_t* pinned = nullptr;  // kStageBytes, allocated on first use
+    uint8_t* pinned = nullptr;      // kStageBytes + kDirectBytes, allocated on first use
+    uint8_t* pinned_dev = nullptr;  // the same as the device addresses it
 };
 
 class ArenaPool {
@@ -164,7 +172,9 @@ public:
         }
         arena_pool().give(a_);
     }
-    int begin(std::initializer_list<size_t> in, std::initializer_list<size_t> out, size_t ws) {
+    // direct: the kernels only write the outputs (never read them back), so small ones may live in
+    // host memory
+    int begin(std::initializer_list<size_t> in, std::initializer_list<size_t> out, size_t ws, bool direct = false) {
         int dev = 0;
         PPOCR_HIP(hipGetDevice(&dev));
         a_ = arena_pool().take(dev);
@@ -194,9 +204,18 @@ public:
         }
         if (!a_->pinned && (in_end_ - in_begin_ <= kStageBytes || out_end_ - in_end_ <= kStageBytes)) {
             void* p = nullptr;
-            if (hipHostMalloc(&p, kStageBytes, hipHostMallocDefault) == hipSuccess) a_->pinned = static_cast<uint8_t*>(p);
-            else (void)hipGetLastError();  // no staging: copies go directly
+            void* d = nullptr;
+            if (hipHostMalloc(&p, kStageBytes + kDirectBytes, hipHostMallocDefault) != hipSuccess) {
+                (void)hipGetLastError();  // no staging: copies go directly
+            } else if (hipHostGetDevicePointer(&d, p, 0) != hipSuccess) {
+                (void)hipGetLastError();
+                (void)hipHostFree(p);
+            } else {
+                a_->pinned = static_cast<uint8_t*>(p);
+                a_->pinned_dev = static_cast<uint8_t*>(d);
+            }
         }
+        direct_ = direct && a_->pinned && out_end_ - in_end_ <= kDirectBytes;
         return PPOCR_OK;
     }
     template <typename T>
@@ -205,7 +224,8 @@ public:
     }
     template <typename T>
     T* out(size_t i) const {
-        return reinterpret_cast<T*>(a_->base + out_[i].first);
+        return reinterpret_cast<T*>(direct_ ? a_->pinned_dev + kStageBytes + (out_[i].first - in_end_)
+                                            : a_->base + out_[i].first);
     }
     uint8_t* ws() const { return a_->base + ws_off_; }
     size_t ws_bytes() const { return ws_bytes_; }
@@ -215,14 +235,30 @@ public:
         size_t i = 0;
         const size_t span = in_end_ - in_begin_;
         const bool staged = a_->pinned && span <= kStageBytes;
+        size_t sent = 0;  // bytes of the stage on their way to the device
         for (const void* src : srcs) {
             const auto [off, n] = in_[i++];
             if (!n || !src) continue;
-            if (staged) std::memcpy(a_->pinned + (off - in_begin_), src, n);
-            else PPOCR_HIP(hipMemcpyAsync(a_->base + off, src, n, hipMemcpyHostToDevice, a_->stream));
+            if (!staged) {
+                PPOCR_HIP(hipMemcpyAsync(a_->base + off, src, n, hipMemcpyHostToDevice, a_->stream));
+                continue;
+            }
+            const size_t at = off - in_begin_;
+            for (size_t d = 0; d < n;) {
+                const size_t len = std::min(n - d, sent + kStagePiece > at + d ? sent + kStagePiece - (at + d) : kStagePiece);
+                std::memcpy(a_->pinned + at + d, static_cast<const uint8_t*>(src) + d, len);
+                d += len;
+                if (at + d >= sent + kStagePiece) {
+                    // whole 16-byte chunks: the slots are 256-byte aligned and padded
+                    const size_t end = align256(at + d) <= span && d == n ? align256(at + d) : (at + d) / 16 * 16;
+                    if (int e = launch_stage_copy(a_->base + in_begin_ + sent, a_->pinned_dev + sent, end - sent, a_->stream))
+                        return e;
+                    sent = end;
+                }
+            }
         }
-        if (staged && span)
-            PPOCR_HIP(hipMemcpyAsync(a_->base + in_begin_, a_->pinned, span, hipMemcpyHostToDevice, a_->stream));
+        if (staged && span > sent)
+            return launch_stage_copy(a_->base + in_begin_ + sent, a_->pinned_dev + sent, span - sent, a_->stream);
         return PPOCR_OK;
     }
     // Copies the outputs back (dsts in the order given to begin; null ones are skipped) and
@@ -230,7 +266,9 @@ public:
     int copy_out(std::initializer_list<void*> dsts) const {
         const size_t span = out_end_ - in_end_;
         const bool staged = a_->pinned && span <= kStageBytes;
-        if (staged) {
+        const uint8_t* from = direct_ ? a_->pinned + kStageBytes : a_->pinned;
+        if (direct_) {
+        } else if (staged) {
             if (span) PPOCR_HIP(hipMemcpyAsync(a_->pinned, a_->base + in_end_, span, hipMemcpyDeviceToHost, a_->stream));
         } else {
             size_t i = 0;
@@ -244,7 +282,7 @@ public:
             size_t i = 0;
             for (void* dst : dsts) {
                 const auto [off, n] = out_[i++];
-                if (n && dst) std::memcpy(dst, a_->pinned + (off - in_end_), n);
+                if (n && dst) std::memcpy(dst, from + (off - in_end_), n);
             }
         }
         return PPOCR_OK;
@@ -258,6 +296,7 @@ private:
     HostArena* a_ = nullptr;
     std::vector<std::pair<size_t, size_t>> in_, out_;  // (offset, bytes)
     size_t in_begin_ = 0, in_end_ = 0, out_end_ = 0, ws_off_ = 0, ws_bytes_ = 0;
+    bool direct_ = false;  // the outputs are in the pinned buffer, after the stage
 };
 
 // Device buffer owned for the duration of a host-pointer call.
@@ -1156,7 +1195,7 @@ int ppocr_rh_decode(const ppocr_rh_t* h, const float* a, const int64_t* line_off
     const size_t wsb = m > 0 ? ws_layout(m, nsplit_for(h, m, cfg)).total : 0;
     const size_t ab = (size_t)(m * h->k) * 4, rb = (size_t)m * 4, ob = (size_t)(lines + 1) * 8;
     HostCall hc;
-    if (int e = hc.begin({ab, ob}, {rb, (size_t)lines * 8, (size_t)lines * 4, idx ? rb : 0, maxprob ? rb : 0}, wsb))
+    if (int e = hc.begin({ab, ob}, {rb, (size_t)lines * 8, (size_t)lines * 4, idx ? rb : 0, maxprob ? rb : 0}, wsb, true))
         return e;
     if (int e = hc.copy_in({a, line_off})) return e;
     if (int e = ppocr_rh_decode_dev(h, hc.in<float>(0), m, hc.in<int64_t>(1), lines, mode,
@@ -1208,7 +1247,7 @@ int ppocr_rh_decode_nct(const ppocr_rh_t* h, const float* x, int64_t lines, int6
     const size_t wsb = m > 0 ? ws_layout(m, nsplit_for(h, m, cfg)).total : 0;
     const size_t xb = (size_t)(m * h->k) * 4, rb = (size_t)m * 4;
     HostCall hc;
-    if (int e = hc.begin({xb}, {rb, (size_t)lines * 8, (size_t)lines * 4, idx ? rb : 0, maxprob ? rb : 0}, wsb))
+    if (int e = hc.begin({xb}, {rb, (size_t)lines * 8, (size_t)lines * 4, idx ? rb : 0, maxprob ? rb : 0}, wsb, true))
         return e;
     if (int e = hc.copy_in({x})) return e;
     if (int e = ppocr_rh_decode_nct_dev(h, hc.in<float>(0), lines, steps, mode, idx ? hc.out<int32_t>(3) : nullptr,

@@ -152,6 +152,10 @@ int launch_build_records(const TileGeom& g, int64_t n, int64_t k, const int8_t* 
 // the library allocates, before its first use.
 int launch_guard_clear(unsigned long long* guard_header, hipStream_t st);
 
+// dst[0 .. bytes) = src (device address of pinned host memory); bytes a multiple of 16, both
+// 16-byte aligned.
+int launch_stage_copy(void* dst, const void* src, size_t bytes, hipStream_t st);
+
 // rec: the records the configuration reads (fp16 for H*, bf16 otherwise); rec_rescue: the
 // bf16 records of the three-term rescue of guarded rows (INT8 heads).
 int launch_logits_mfma(int cfg, const TileGeom& tg, const uint8_t* rec, const uint8_t* rec_rescue, const float* a,

@@ -215,4 +215,20 @@ int launch_build_records(const TileGeom& g, int64_t n, int64_t k, const int8_t* 
     return PPOCR_OK;
 }
 
+// Pinned host memory to device memory, bound by PCIe: a thread per 16 bytes, every load of the
+// piece in flight at once.
+__global__ __launch_bounds__(256) void stage_copy_kernel(u32x4* __restrict__ dst, const u32x4* __restrict__ src, int n) {
+    const int x = blockIdx.x * 256 + threadIdx.x;
+    if (x < n) dst[x] = src[x];
+}
+
+int launch_stage_copy(void* dst, const void* src, size_t bytes, hipStream_t st) {
+    if (bytes == 0) return PPOCR_OK;
+    if (bytes % 16 != 0 || bytes > (1u << 30)) return fail(PPOCR_ERR_INVALID_ARG, "RecHeadHip: bad staging copy");
+    const int n = (int)(bytes / 16);
+    stage_copy_kernel<<<(n + 255) / 256, 256, 0, st>>>(static_cast<u32x4*>(dst), static_cast<const u32x4*>(src), n);
+    PPOCR_HIP(hipGetLastError());
+    return PPOCR_OK;
+}
+
 }  // namespace ppocr

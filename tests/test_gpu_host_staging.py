@@ -1,0 +1,33 @@
+"""Host decode calls whose inputs end around the staging pieces (512 KB), leave the stage (4 MB),
+and whose results leave the pinned buffer (256 KB): the bits of one device call."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def test_host_decode_across_the_staging_sizes(rh, orc):
+    from ppocr_rechead.hip import DeviceArray, synchronize
+    rng = np.random.default_rng(5)
+    w = (rng.standard_normal((200, 120)) * 0.05).astype(np.float32)
+    q, s = orc.pack_int8(w)
+    head = rh.RecHead(qw=rh.QuantizedWeight(q, s), bias=np.zeros(200, np.float32))
+    L = rh._lib.lib()
+    for m in (1, 1092, 1093, 2184, 2185, 8737, 8738, 24000, 1092):
+        a = rng.standard_normal((m, 120)).astype(np.float32)
+        off = np.array([0, m // 3, m], np.int64)
+        got = head.decode(a, off, 2)
+        da, doff = DeviceArray.from_numpy(a), DeviceArray.from_numpy(off)
+        di, dm, dq = DeviceArray((m,), np.int32), DeviceArray((m,), np.float32), DeviceArray((m,), np.int32)
+        dl, ds = DeviceArray((2,), np.int64), DeviceArray((2,), np.float32)
+        ws = head.workspace_bytes(m, 2)
+        dw = DeviceArray((ws,), np.uint8)
+        rh._check(L.ppocr_rh_decode_dev(head.handle, da.p, m, doff.p, 2, 2, di.p, dm.p, dq.p, dl.p, ds.p, dw.p, ws, None))
+        synchronize()
+        assert np.array_equal(got["idx"], di.numpy()), m
+        assert np.array_equal(got["maxprob"], dm.numpy()), m
+        assert np.array_equal(got["score"], ds.numpy()), m
+        assert [len(x) for x in got["seqs"]] == dl.numpy().tolist(), m
+        for d in (da, doff, di, dm, dq, dl, ds, dw):
+            d.free()
+    head.close()
