@@ -1484,11 +1484,13 @@ int neck_create(const NeckHost& nh, int device, ppocr_rn_t** out) {
     }
     h->d_weights = static_cast<float*>(p);
     h->device_bytes = (size_t)total * 4;
-    std::vector<float> host((size_t)total, 0.0f);
+    int64_t uploaded = 0;  // the parts without host data come last
+    for (const auto& pt : parts) uploaded += pt.first ? (pt.second + 3) / 4 * 4 : 0;
+    std::vector<float> host((size_t)uploaded, 0.0f);
     std::vector<const float*> dev_ptr;
-    int64_t off = 0, uploaded = 0;  // the parts without host data come last
+    int64_t off = 0;
     for (const auto& pt : parts) {
-        if (pt.first) std::memcpy(host.data() + off, pt.first, (size_t)pt.second * 4), uploaded = off + pt.second;
+        if (pt.first) std::memcpy(host.data() + off, pt.first, (size_t)pt.second * 4);
         dev_ptr.push_back(h->d_weights + off);
         off += (pt.second + 3) / 4 * 4;
     }
