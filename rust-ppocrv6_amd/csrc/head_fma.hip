@@ -29,10 +29,13 @@ constexpr int LST = KC + 4;
 constexpr size_t kFmaLdsFloats = 2 * (size_t)(BM + BN) * LST;
 static_assert(BM == 128 && BN == 128 && KC == 16, "the thread mappings below");
 
-// Where the operands may be read 4 values of k at a time: k a multiple of 4 and the row
-// starts aligned (16 bytes for floats, 4 for int8).
-bool vec_rows(const float* p, int64_t k) { return k % 4 == 0 && reinterpret_cast<uintptr_t>(p) % 16 == 0; }
-bool vec_rows(const int8_t* p, int64_t k) { return k % 4 == 0 && reinterpret_cast<uintptr_t>(p) % 4 == 0; }
+// Where the operands may be read 4 values of k at a time: k a multiple of 4, the row starts
+// aligned (16 bytes for floats, 4 for int8), and 128 rows within 32-bit offsets.
+constexpr int64_t kOffsetK = 1 << 24;
+bool vec_rows(const float* p, int64_t k) { return k % 4 == 0 && k <= kOffsetK && reinterpret_cast<uintptr_t>(p) % 16 == 0; }
+bool vec_rows(const int8_t* p, int64_t k) { return k % 4 == 0 && k <= kOffsetK && reinterpret_cast<uintptr_t>(p) % 4 == 0; }
+// Most classes whose output rows r and r + 4 are addressed by 32-bit offsets.
+constexpr int kOffsetClasses = 1 << 29;
 
 // Row of slot j: contiguous rows, or (GATHER) an entry of the precision guard's row list of
 // another kernel's pass (checked, not trusted: an entry outside [0, m) is skipped); -1: none.
@@ -199,7 +202,9 @@ __global__ __launch_bounds__(256, EPI == EPI_STATS || GATHER ? 2 : 3) void head_
         struct Step {
             int n0, x;
         };
-        auto next = [&](Step q_) { return q_.x + 1 < nk ? Step{q_.n0, q_.x + 1} : Step{q_.n0 + BN, 0}; };
+        auto next = [&](Step q_) {  // past the last tile n0 stays at or past c1
+            return q_.x + 1 < nk ? Step{q_.n0, q_.x + 1} : Step{q_.n0 < c1 ? q_.n0 + BN : q_.n0, 0};
+        };
         struct Frag {
             f32x4 a, w[4];
         };
@@ -318,9 +323,8 @@ __global__ __launch_bounds__(256, EPI == EPI_STATS || GATHER ? 2 : 3) void head_
                     return __builtin_amdgcn_exp2f(fmaf(acc[t][r], csc[t] * kLog2e, cbi[t] * kLog2e) - s_max[lr]) *
                            s_inv[lr];
                 };
-                // a whole tile: one 32-bit lane offset (4 h rows and i classes; the launcher bounds
-                // n) from a row address that is the same in every lane
-                const bool all = !GATHER && n0 + BN <= c1 && m0 + BM <= m;
+                // a whole tile: one 32-bit lane offset (4 h rows and i classes) from a row address that is the same in every lane
+                const bool all = !GATHER && n <= kOffsetClasses && n0 + BN <= c1 && m0 + BM <= m;
                 unsigned lo = (unsigned)(4 * h) * (unsigned)n + (unsigned)i;
                 asm volatile("" : "+v"(lo));  // not before the products, where it would hold registers
                 float* obase = out + (m0 + 32 * wave) * n + n0;
@@ -382,7 +386,7 @@ __global__ __launch_bounds__(256, EPI == EPI_STATS || GATHER ? 2 : 3) void head_
 }
 
 int check_fma_args(int64_t m, int64_t n, int64_t k) {
-    if (n > 0x0fffffff || k > 0x7fffffff - KC) return fail(PPOCR_ERR_INVALID_ARG, "MatMulQuantizedB: shape too large");
+    if (n > 0x7fffffff - BN || k > 0x7fffffff - KC) return fail(PPOCR_ERR_INVALID_ARG, "MatMulQuantizedB: shape too large");
     if ((m + BM - 1) / BM > 65535) return fail(PPOCR_ERR_INVALID_ARG, "MatMulQuantizedB: m too large for the fp32 path");
     return PPOCR_OK;
 }
