@@ -1287,67 +1287,11 @@ struct NeckHost {
     const float *lnf_w = nullptr, *lnf_b = nullptr;
 };
 
-// fp16 planes of W^T for the tail's fp16-halves GEMMs: [2][N][kp], the nearest half of each
-// weight, then the nearest half of what it leaves, k padded with zeros.
-std::vector<uint16_t> neck_half_planes(const float* w, int64_t K, int64_t N) {
-    const int64_t kp = neck_f16_kp((int)K);
-    std::vector<uint16_t> out((size_t)(2 * N * kp), 0);
-    for (int64_t k = 0; k < K; ++k)
-        for (int64_t c = 0; c < N; ++c) {
-            const float x = w[k * N + c];
-            const _Float16 hi = (_Float16)x;
-            const _Float16 lo = (_Float16)(x - (float)hi);
-            out[(size_t)(c * kp + k)] = __builtin_bit_cast(uint16_t, hi);
-            out[(size_t)((N + c) * kp + k)] = __builtin_bit_cast(uint16_t, lo);
-        }
-    return out;
-}
-
 // Column of the padded qkv row (or attention row) that holds column c of the model's:
 // part c / D (q, k, v), head (c % D) / 15, value c % 15 -> 128 part + 16 head + value.
 int64_t neck_pad_col(int64_t c) {
     const int64_t part = c / kNeckDim, r = c % kNeckDim;
     return 128 * part + 16 * (r / kNeckHeadDim) + r % kNeckHeadDim;
-}
-
-// fc1's and fc2's weights in the fused MLP kernel's staging order (NeckBlockDev::mlp_h),
-// each weight times 2^e1 (fc1) or 2^e2 (fc2), exact, before the split, so that the low
-// halves stay above fp16's subnormals.  fc2's contraction index runs in the order
-// K' = 32 T + 16 q + 8 h + e <-> hidden unit 32 T + 16 q + 8 (e / 4) + 4 h + e % 4, the
-// order in which fc1's transposed MFMA output leaves the hidden values in registers.
-std::vector<uint16_t> neck_mlp_tiles(const ppocr_rn_block_t& b, int64_t D, int64_t H, int e1, int e2) {
-    constexpr int kTiles = 8, kTileHalves = 16384;  // 32 KB per tile
-    std::vector<uint16_t> out((size_t)kTiles * kTileHalves, 0);
-    auto split = [](float v, uint16_t* hi, uint16_t* lo) {
-        const _Float16 h = (_Float16)v;
-        *hi = __builtin_bit_cast(uint16_t, h);
-        *lo = __builtin_bit_cast(uint16_t, (_Float16)(v - (float)h));
-    };
-    for (int T = 0; T < kTiles; ++T) {
-        uint16_t* t = out.data() + (size_t)T * kTileHalves;
-        // fc1: [plane][chunk c (16)][unit u (32)][8]: unit 32 T + u, k = 8 c + e
-        for (int c = 0; c < 16; ++c)
-            for (int u = 0; u < 32; ++u)
-                for (int e = 0; e < 8; ++e) {
-                    const int64_t unit = 32 * T + u, k = 8 * c + e;
-                    if (unit >= H || k >= D) continue;
-                    split(std::ldexp(b.fc1_w[k * H + unit], e1), &t[((size_t)c * 32 + u) * 8 + e],
-                          &t[((size_t)(16 + c) * 32 + u) * 8 + e]);
-                }
-        // fc2: [plane][chunk c (4)][column (128)][8]: contraction position K' = 32 T + 8 c + e
-        uint16_t* t2 = t + 8192;
-        for (int c = 0; c < 4; ++c)
-            for (int col = 0; col < 128; ++col)
-                for (int e = 0; e < 8; ++e) {
-                    const int kp = 32 * T + 8 * c + e;
-                    const int ee = kp & 7, hh = (kp >> 3) & 1, q = (kp >> 4) & 1;
-                    const int64_t unit = 32 * T + 16 * q + 8 * (ee >> 2) + 4 * hh + (ee & 3);
-                    if (unit >= H || col >= D) continue;
-                    split(std::ldexp(b.fc2_w[unit * D + col], e2), &t2[((size_t)c * 128 + col) * 8 + e],
-                          &t2[((size_t)(4 + c) * 128 + col) * 8 + e]);
-                }
-    }
-    return out;
 }
 
 // Whether the weights keep every operand of the tail's GEMMs and attention inside fp16's range,
@@ -1439,35 +1383,20 @@ int neck_create(const NeckHost& nh, int device, ppocr_rn_t** out) {
     }
     parts.push_back({nh.lnf_w, D});
     parts.push_back({nh.lnf_b, D});
-    // the fp16 planes of each block's four weights, as float-sized parts after the rest
     int exps[kNeckMaxBlocks][kNeckExps] = {};
     const bool f16 = neck_f16_bounds_ok(nh, exps);
-    std::vector<std::vector<uint16_t>> planes;
     std::vector<std::vector<float>> padded_bias;
     if (f16) {
-        for (const ppocr_rn_block_t& b : nh.blocks) {
-            const size_t bi = (size_t)(&b - nh.blocks.data());
-            // qkv's columns and proj's rows padded per head to 16 (zeros at d = 15)
-            std::vector<float> qp((size_t)D * kNeckQkvPad, 0.0f), pp((size_t)kNeckAttPad * D, 0.0f);
-            for (int64_t k = 0; k < D; ++k)
-                for (int64_t c = 0; c < 3 * D; ++c)
-                    qp[(size_t)(k * kNeckQkvPad + neck_pad_col(c))] = b.qkv_w[k * 3 * D + c];
-            for (int64_t k = 0; k < D; ++k) std::memcpy(&pp[(size_t)(neck_pad_col(k) * D)], b.proj_w + k * D, (size_t)D * 4);
-            planes.push_back(neck_half_planes(qp.data(), D, kNeckQkvPad));
-            planes.push_back(neck_half_planes(pp.data(), kNeckAttPad, D));
-            planes.push_back(neck_mlp_tiles(b, D, H, exps[bi][3], exps[bi][4]));
-        }
-        for (const auto& pl : planes)
-            parts.push_back({reinterpret_cast<const float*>(pl.data()), (int64_t)(pl.size() / 2)});
+        // qkv's bias in the padded column order (zeros at d = 15), then each block's fp16 planes,
+        // built on the device (no host data)
         for (const ppocr_rn_block_t& b : nh.blocks) {
             std::vector<float> bp(kNeckQkvPad, 0.0f);
             for (int64_t c = 0; c < 3 * D; ++c) bp[(size_t)neck_pad_col(c)] = b.qkv_b[c];
             padded_bias.push_back(std::move(bp));
         }
         for (const auto& bp : padded_bias) parts.push_back({bp.data(), (int64_t)bp.size()});
-        // the block kernels' planes, built on the device (no host data)
         for (size_t i = 0; i < nh.blocks.size(); ++i)
-            for (int halves : kNeckFragHalves) parts.push_back({nullptr, halves / 2});
+            for (int halves : kNeckPlaneHalves) parts.push_back({nullptr, halves / 2});
     }
     int64_t total = 0;
     for (const auto& pt : parts) total += (pt.second + 3) / 4 * 4;  // each part 16-byte aligned
@@ -1525,9 +1454,6 @@ int neck_create(const NeckHost& nh, int device, ppocr_rn_t** out) {
     nd.f16 = f16;
     for (size_t i = 0; f16 && i < nh.blocks.size(); ++i) {
         NeckBlockDev& b = nd.block[i];
-        b.qkv_h = reinterpret_cast<const uint16_t*>(dev_ptr[q++]);
-        b.proj_h = reinterpret_cast<const uint16_t*>(dev_ptr[q++]);
-        b.mlp_h = reinterpret_cast<const uint16_t*>(dev_ptr[q++]);
         b.attn_eq = exps[i][0];
         b.attn_ek = exps[i][1];
         b.attn_ev = exps[i][2];
@@ -1542,8 +1468,9 @@ int neck_create(const NeckHost& nh, int device, ppocr_rn_t** out) {
     for (size_t i = 0; f16 && i < nh.blocks.size(); ++i) nd.block[i].qkv_bp = dev_ptr[q++];
     for (size_t i = 0; f16 && i < nh.blocks.size(); ++i) {
         NeckBlockDev& b = nd.block[i];
-        for (const uint16_t** f : {&b.qkv_f, &b.proj_f, &b.fc1_f, &b.fc2_f}) *f = reinterpret_cast<const uint16_t*>(dev_ptr[q++]);
-        if (int e = launch_neck_fragments(b, nullptr)) return e;
+        for (const uint16_t** f : {&b.qkv_h, &b.proj_h, &b.mlp_h, &b.qkv_f, &b.proj_f, &b.fc1_f, &b.fc2_f})
+            *f = reinterpret_cast<const uint16_t*>(dev_ptr[q++]);
+        if (int e = launch_neck_planes(b, nullptr)) return e;
     }
     if (f16) PPOCR_HIP(hipStreamSynchronize(nullptr));
     *out = h.release();

@@ -756,24 +756,60 @@ __global__ __launch_bounds__(kThreads, 2) void neck_block_kernel(
     }
 }
 
-// One half of a plane pair's values: thread x the value (tile, step, lane, j) of W [K][N] times
-// mul.  PAD 1: W's columns, padded per head to 16 (qkv); 2: its rows (proj).
+// ---------------------------------------------------------------- planes, at creation
+// (On the host, without half conversions in hardware, these took 3 ms of a tail's creation.)
+__device__ __forceinline__ void put_halves(float v, uint16_t* hi, uint16_t* lo) {
+    const _Float16 h = (_Float16)v;
+    *hi = __builtin_bit_cast(uint16_t, h);
+    *lo = __builtin_bit_cast(uint16_t, (_Float16)(v - (float)h));
+}
+// The model's index of index c padded per head to 16 (qkv's columns, proj's contraction), or one
+// past any.
+__device__ __forceinline__ int unpad(int c) {
+    const int d = c % 16;
+    return d < kNeckHeadDim ? c / 128 * D + c % 128 / 16 * kNeckHeadDim + d : INT32_MAX;
+}
+
+// The planes in operand order: thread x the value (tile, step, lane, j) of W [K][N] times mul.
+// PAD 1: W's columns padded per head (qkv); 2: its rows (proj).
 template <int PAD>
 __global__ __launch_bounds__(256) void neck_fragments_kernel(const float* __restrict__ w, int K, int N, int steps, float mul,
                                                              uint16_t* __restrict__ out) {
     const int x = blockIdx.x * 256 + threadIdx.x, j = x & 7, lane = (x >> 3) & 63, ts = x >> 9;
     int col = 16 * (ts / steps) + lane % 16, k = 32 * (ts % steps) + 8 * (lane / 16) + j;
-    auto unpad = [](int c) {
-        const int d = c % 16;
-        return d < kNeckHeadDim ? c / 128 * D + c % 128 / 16 * kNeckHeadDim + d : INT32_MAX;
-    };
     if (PAD == 1) col = unpad(col);
     if (PAD == 2) k = unpad(k);
-    const float v = col < N && k < K ? w[k * N + col] * mul : 0.0f;
-    const _Float16 hi = (_Float16)v;
     uint16_t* f = out + (size_t)ts * kTileHalves + lane * 8 + j;
-    f[0] = __builtin_bit_cast(uint16_t, hi);
-    f[512] = __builtin_bit_cast(uint16_t, (_Float16)(v - (float)hi));
+    put_halves(col < N && k < K ? w[k * N + col] * mul : 0.0f, f, f + 512);
+}
+
+// The planes [2][columns][128] of the separate kernels' GEMMs, a thread per value; PAD as above.
+template <int PAD>
+__global__ __launch_bounds__(256) void neck_columns_kernel(const float* __restrict__ w, int K, int N, int columns,
+                                                           uint16_t* __restrict__ out) {
+    const int x = blockIdx.x * 256 + threadIdx.x;
+    if (x >= columns * 128) return;
+    const int col = PAD == 1 ? unpad(x / 128) : x / 128, k = PAD == 2 ? unpad(x % 128) : x % 128;
+    put_halves(col < N && k < K ? w[k * N + col] : 0.0f, out + x, out + columns * 128 + x);
+}
+
+// The staging order of the separate kernels' MLP (NeckBlockDev::mlp_h): thread x entry x % 4096 of
+// tile x / 4096, of fc1's part and of fc2's.  fc2's contraction position 32 T + 16 q + 8 h + e
+// holds hidden unit 32 T + 16 q + 8 (e / 4) + 4 h + e % 4, the order in which fc1's transposed
+// MFMA output leaves the hidden values in registers.
+__global__ __launch_bounds__(256) void neck_mlp_tiles_kernel(const float* __restrict__ fc1, const float* __restrict__ fc2,
+                                                             float mul1, float mul2, uint16_t* __restrict__ out) {
+    const int x = blockIdx.x * 256 + threadIdx.x, T = x >> 12, n = x & 4095, e = n & 7;
+    uint16_t* t = out + (size_t)T * 16384;
+    {  // [plane][chunk (16)][unit (32)][8]
+        const int unit = 32 * T + ((n >> 3) & 31), k = 8 * (n >> 8) + e;
+        put_halves(unit < H && k < D ? fc1[k * H + unit] * mul1 : 0.0f, t + n, t + 4096 + n);
+    }
+    {  // [plane][chunk (4)][column (128)][8]
+        const int col = (n >> 3) & 127, c = n >> 10;
+        const int unit = 32 * T + 16 * (c >> 1) + 8 * (e >> 2) + 4 * (c & 1) + (e & 3);
+        put_halves(unit < H && col < D ? fc2[unit * D + col] * mul2 : 0.0f, t + 8192 + n, t + 12288 + n);
+    }
 }
 
 template <int R>
@@ -806,16 +842,18 @@ int go(const NeckDev& nk, const float* x_in, const float* shortcut, int64_t m, c
 
 }  // namespace
 
-int launch_neck_fragments(const NeckBlockDev& k, hipStream_t st) {
-    auto run = [&](auto kern, const float* w, int K, int N, int tiles, int steps, int e, const uint16_t* out) -> int {
-        kern<<<tiles * steps * 2, 256, 0, st>>>(w, K, N, steps, std::ldexp(1.0f, e), const_cast<uint16_t*>(out));
-        PPOCR_HIP(hipGetLastError());
-        return PPOCR_OK;
-    };
-    if (int e = run(neck_fragments_kernel<1>, k.qkv_w, D, 3 * D, 24, 4, k.qkv_e, k.qkv_f)) return e;
-    if (int e = run(neck_fragments_kernel<2>, k.proj_w, D, D, 8, 4, k.proj_e, k.proj_f)) return e;
-    if (int e = run(neck_fragments_kernel<0>, k.fc1_w, D, H, 16, 4, k.mlp_e1, k.fc1_f)) return e;
-    return run(neck_fragments_kernel<0>, k.fc2_w, H, D, 8, 8, k.mlp_e2, k.fc2_f);
+int launch_neck_planes(const NeckBlockDev& k, hipStream_t st) {
+    auto mut = [](const uint16_t* p) { return const_cast<uint16_t*>(p); };
+    auto mul = [](int e) { return std::ldexp(1.0f, e); };
+    neck_columns_kernel<1><<<kNeckQkvPad / 2, 256, 0, st>>>(k.qkv_w, D, 3 * D, kNeckQkvPad, mut(k.qkv_h));
+    neck_columns_kernel<2><<<D / 2, 256, 0, st>>>(k.proj_w, D, D, D, mut(k.proj_h));
+    neck_mlp_tiles_kernel<<<8 * 16, 256, 0, st>>>(k.fc1_w, k.fc2_w, mul(k.mlp_e1), mul(k.mlp_e2), mut(k.mlp_h));
+    neck_fragments_kernel<1><<<24 * 4 * 2, 256, 0, st>>>(k.qkv_w, D, 3 * D, 4, mul(k.qkv_e), mut(k.qkv_f));
+    neck_fragments_kernel<2><<<8 * 4 * 2, 256, 0, st>>>(k.proj_w, D, D, 4, mul(k.proj_e), mut(k.proj_f));
+    neck_fragments_kernel<0><<<16 * 4 * 2, 256, 0, st>>>(k.fc1_w, D, H, 4, mul(k.mlp_e1), mut(k.fc1_f));
+    neck_fragments_kernel<0><<<8 * 8 * 2, 256, 0, st>>>(k.fc2_w, H, D, 8, mul(k.mlp_e2), mut(k.fc2_f));
+    PPOCR_HIP(hipGetLastError());
+    return PPOCR_OK;
 }
 
 int launch_neck_fused(const NeckDev& nk, const float* x_in, const float* shortcut, int64_t m, const int64_t* line_off,
