@@ -666,17 +666,17 @@ Guard make_guard(const ppocr_rh* h, int cfg, const WsLayout& L, uint8_t* ws, int
 const uint8_t* rec_of(const ppocr_rh* h, int cfg) { return cfg_is_f16(cfg) ? h->d_rec_h : h->d_rec; }
 
 // Projection + softmax statistics + merge (+ the CTC collapse with `ctc`), on device pointers.
-// line_len > 0: d_a is channels-first, [m / line_len][k][line_len].  epoch: the guard list's, which
-// the merge leaves empty under it.
+// line_len > 0: d_a is channels-first, [m / line_len][k][line_len].  writer_epoch: that of the
+// probabilities' writer that follows in the same call (0: none), see Guard.
 int run_stats(const ppocr_rh* h, int cfg, const float* d_a, int64_t m, int32_t* d_idx, float* d_maxprob,
               float* d_row_max, float* d_row_inv, uint8_t* ws, hipStream_t st, const CtcOut* ctc = nullptr,
-              int64_t line_len = 0, unsigned* epoch = nullptr) {
+              int64_t line_len = 0, unsigned writer_epoch = 0) {
     const int nsplit = nsplit_for(h, m, cfg);
     const WsLayout L = ws_layout(m, nsplit);
     Partial* part = reinterpret_cast<Partial*>(ws + L.part);
     if (cfg >= 0) {
-        const Guard g = make_guard(h, cfg, L, ws, m);
-        if (epoch) *epoch = g.epoch;
+        Guard g = make_guard(h, cfg, L, ws, m);
+        g.writer_epoch = writer_epoch;
         return launch_stats_mfma(cfg, h->geom, rec_of(h, cfg), h->d_rec, d_a, m, h->n, h->k, nsplit, part, &g, d_idx, d_maxprob, d_row_max, d_row_inv, ctc, st, line_len);
     }
     if (int e = launch_stats_fma(h->d_q, h->d_w, h->d_scale, h->d_bias, d_a, m, h->n, h->k, nsplit, part, st, line_len))
@@ -1068,13 +1068,13 @@ int ppocr_rh_probs_dev(const ppocr_rh_t* h, const float* d_a, int64_t m, int mod
     if (int e = ws.get(d_workspace, workspace_bytes, L.total, st, "RecHeadHip")) return e;
     float* rmax = reinterpret_cast<float*>(ws.p + L.row_max);
     float* rinv = reinterpret_cast<float*>(ws.p + L.row_inv);
-    unsigned epoch = 0;
-    if (int e = run_stats(h, cfg, d_a, m, nullptr, nullptr, rmax, rinv, ws.p, st, nullptr, 0, &epoch)) return e;
-    if (cfg < 0)
+    if (cfg < 0) {
+        if (int e = run_stats(h, cfg, d_a, m, nullptr, nullptr, rmax, rinv, ws.p, st)) return e;
         return launch_probs_fma(h->d_q, h->d_w, h->d_scale, h->d_bias, d_a, m, h->n, h->k, rmax, rinv, d_probs, st);
+    }
     Guard g = make_guard(h, cfg, L, ws.p, m);
-    g.epoch = epoch;
     g.emptied = true;
+    if (int e = run_stats(h, cfg, d_a, m, nullptr, nullptr, rmax, rinv, ws.p, st, nullptr, 0, g.epoch)) return e;
     return launch_probs_mfma(cfg, h->geom, rec_of(h, cfg), h->d_rec, d_a, m, h->n, h->k, rmax, rinv, d_probs, &g, st);
 }
 

@@ -102,7 +102,10 @@ int rows_cfg(const RowsLaunch& x, int epi, unsigned grid, hipStream_t st);
 // 64-bit header holds (epoch << 32) | count.  Every call draws a new epoch; the first
 // append of a call installs it (count 0), and a header with another epoch counts as empty,
 // so a fresh or stale workspace needs no reset.  Paths that end with a merge kernel reset
-// the header to (epoch, 0) there, so a replay of the same call (same epoch) starts empty.
+// the header to (epoch, 0) there, so a replay of the same call (same epoch) starts empty.  A
+// call of two passes (statistics, then the probabilities' writer) draws an epoch for each:
+// the merge between them writes (the writer's epoch, 0), so the writer starts empty without a
+// reset launch, and the list it leaves is of another epoch than a replay's statistics pass.
 // The statistics pass may skip the reference shift of the softmax sum (stats_noref) when
 // the head bounds its logits: its rescue pass, which keeps the shift, then also takes the
 // rows whose logits are not proven to lie in [-kLogitBound, kLogitBound] (GuardLimits).
@@ -119,9 +122,13 @@ struct Guard {
     bool stats_noref;
     const FmaWeights& fma;  // the head's fp32 weights, for a rescue in fp32 FMA
     uint8_t* skip;          // a byte per 128 rows: the statistics pass's skipped row blocks
-    // the list was emptied earlier in this call under the same epoch (by the statistics
-    // merge before a probabilities pass): no reset launch
+    // statistics: the epoch the merge leaves the empty list under, when a writer with that
+    // epoch follows (0: the pass's own)
+    unsigned writer_epoch = 0;
+    // writer: the statistics merge of the same call left the list empty under this epoch (no
+    // reset launch)
     bool emptied = false;
+    unsigned merge_epoch() const { return writer_epoch ? writer_epoch : epoch; }
 };
 
 // Supported group counts (k = 113..120 and k = 73..80, the PP-OCRv6 small and tiny heads).
@@ -220,7 +227,7 @@ int launch_rescue_fma(int epi, const FmaWeights& fw, const float* a, int64_t m, 
 
 // Merge the per-chunk partials of each row: argmax index, max probability, and (when
 // row_max/row_inv are non-null) the row's log2-domain maximum and 1/sum for a probs pass.
-// With `guard`, the merge also resets the guard header to (epoch, 0) (see Guard).
+// With `guard`, the merge also resets the guard header to (merge_epoch, 0) (see Guard).
 int launch_merge_stats(const Partial* part, int64_t m, int nsplit, int32_t* idx, float* maxprob, float* row_max, float* row_inv,
                        const Guard* guard, hipStream_t st);
 

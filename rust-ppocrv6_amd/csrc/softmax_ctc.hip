@@ -428,7 +428,7 @@ int launch_merge_stats(const Partial* part, int64_t m, int nsplit,
     if (blocks > 0x7fffffffLL) return fail(PPOCR_ERR_INVALID_ARG, "RecHeadHip: m too large");
     merge_stats_kernel<<<(unsigned)blocks, 256, 0, st>>>(part, m, nsplit, idx, maxprob, row_max,
                                                          row_inv, guard ? guard->header : nullptr,
-                                                         guard ? guard->epoch : 0u);
+                                                         guard ? guard->merge_epoch() : 0u);
     PPOCR_HIP(hipGetLastError());
     return PPOCR_OK;
 }
@@ -451,7 +451,7 @@ int launch_merge_ctc(const Partial* part, int64_t m, int nsplit,
     if (ctc.lines > 0x7fffffffLL) return fail(PPOCR_ERR_INVALID_ARG, "CtcDecode: too many lines");
     merge_ctc_kernel<<<(unsigned)ctc.lines, 1024, 0, st>>>(part, m, nsplit, ctc.line_off, ctc.lines,
                                                        ctc.blank, idx, maxprob, ctc.seq, ctc.seq_len, ctc.score,
-                                                       guard ? guard->header : nullptr, guard ? guard->epoch : 0u,
+                                                       guard ? guard->header : nullptr, guard ? guard->merge_epoch() : 0u,
                                                        ctc.line_len);
     PPOCR_HIP(hipGetLastError());
     return PPOCR_OK;
