@@ -1138,20 +1138,23 @@ __global__ __launch_bounds__(64 * (kWriterWaves + 1), 1) void rows_w_kernel(
                     v[r] = __builtin_amdgcn_exp2f(fmaf(acc[r], c0, c1) - rmax[r]) * rinv[r];
                 }
             }
-            if (!GATHER && n <= kBufferClasses) {
-                // one 32-bit offset per row from the wave's first row; the buffer ends with the
-                // batch, so rows past it are dropped by the bounds check, and so are classes past
-                // n, moved past any end.  A branch per row instead made the compiler wait for the
-                // stores in flight: a batch that is no multiple of 128 rows waited for its last
-                // row block (12000 rows in one chunk: 94 row blocks 381 us, whole ones 326).
+            if (all_valid && tt * 32 + 32 <= n) {
+#pragma unroll
+                for (int r = 0; r < 16; ++r) out[(int64_t)orow[r] * n + col] = v[r];
+            } else if (!GATHER && n <= kBufferClasses) {
+                // The last rows or classes: one 32-bit offset per row from the wave's first row; the
+                // buffer ends with the batch, so rows past it are dropped by the bounds check, and
+                // so are classes past n, moved past any end.  A branch per row instead made the
+                // compiler wait for the stores in flight: a batch that is no multiple of 128 rows
+                // waited for its last row block (12000 rows of the 18710-class head in one chunk
+                // took 381 us with its row branches, 326 as 93 whole row blocks, 338 so).  Whole
+                // tiles as well through the buffer took longer: 6144 rows of a 6906-class head 39
+                // us, 36 so.
                 const unsigned o = col < n ? ((unsigned)(4 * h) * (unsigned)n + (unsigned)col) * 4u : 0xFFFFFFFFu;
                 const unsigned add = col < n ? 4u * (unsigned)n : 0u;
 #pragma unroll
                 for (int r = 0; r < 16; ++r)
                     __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v[r]), obuf, o + (8 * (r >> 2) + (r & 3)) * add, 0, 0);
-            } else if (all_valid && tt * 32 + 32 <= n) {
-#pragma unroll
-                for (int r = 0; r < 16; ++r) out[(int64_t)orow[r] * n + col] = v[r];
             } else if (col < n) {
 #pragma unroll
                 for (int r = 0; r < 16; ++r)

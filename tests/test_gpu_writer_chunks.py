@@ -13,7 +13,9 @@ from test_gpu_random_shapes import _head
 pytestmark = pytest.mark.gpu
 
 CASES = [(1, 18710), (129, 18710), (500, 33), (641, 1), (2177, 2049), (2689, 2049), (4097, 4001), (9089, 257),
-         (16513, 65), (33025, 97)]
+         (16513, 65), (33025, 97),
+         # whole row blocks, with whole tiles alone and with a last tile of some classes
+         (128, 64), (256, 33), (2304, 2080)]
 
 
 @pytest.mark.parametrize("m,n", CASES)
