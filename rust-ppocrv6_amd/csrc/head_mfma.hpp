@@ -971,6 +971,12 @@ constexpr int writer_ring() {
     return 2 + 63 / stage_wave_ops<REC>() < 8 ? 2 + 63 / stage_wave_ops<REC>() : 8;
 }
 
+// Most classes whose 32-row blocks are addressed by 32-bit offsets.
+constexpr int kBufferClasses = 1 << 24;
+// Fraction of its chunk, in 2^-16, by which a writer workgroup's starting tile lies past that
+// of the workgroup before it: in one chunk per row block, in several.
+constexpr unsigned kStartStepOne = 25033, kStartStepSeveral = 5063;
+
 // Projection writing logits (EPI 0) or softmax probabilities (EPI 1).  A workgroup owns
 // 32 * NC activation rows.  Waves 0..NC-1 are consumers, one 32-row block each; wave NC is
 // the producer: it keeps a ring of R weight tiles in LDS, R - 1 tiles ahead of the
@@ -980,8 +986,6 @@ constexpr int writer_ring() {
 // class of 16 rows, so each store instruction writes 32 consecutive classes of two rows.
 // GATHER: the rows are the entries of the guard list (the rescue of guarded rows); a
 // workgroup then takes several row blocks and the producer streams the tiles once per block.
-// Most classes whose 32-row blocks are addressed by 32-bit offsets.
-constexpr int kBufferClasses = 1 << 24;
 template <int C, int G, int EPI, bool GATHER>
 __global__ __launch_bounds__(64 * (kWriterWaves + 1), 1) void rows_w_kernel(
     const float* __restrict__ a, int64_t m, int k, int vec, const uint8_t* __restrict__ rec, int tiles, int n,
@@ -1011,11 +1015,15 @@ __global__ __launch_bounds__(64 * (kWriterWaves + 1), 1) void rows_w_kernel(
     // with the write stream running, L2 read latency rose from about 300 cycles (one tile
     // re-read) to 1450 and write latency from 320 to 1000 (TCP_TCC_*_REQ_LATENCY), and the
     // logits kernel took 843 us instead of 648 (dense batch, same box).
-    // The starts of an XCD's workgroups (ids 8 apart) follow the golden ratio (8 x 5063 / 2^16 =
-    // 0.618), spread over the chunk whatever its length; the XCDs' own start an eighth of that
-    // apart.  (149 tiles per row block, as before, put the starts of chunks of 37, 74 or 147 tiles
-    // one or two tiles apart: 30720 rows in 4 chunks 779 us, 649 so.)
-    const int rot = (int)(((int64_t)((blockIdx.x * 5063u) & 0xffffu) * ntiles) >> 16);
+    // The starts are fractions of the chunk, whatever its length, and follow the golden ratio: in
+    // one chunk per row block from one workgroup to the next (0.382), in several from one
+    // workgroup of an XCD to its next (ids 8 apart: 8 x 5063 / 2^16 = 0.618), the XCDs an eighth
+    // of that apart.  Logits in us, 18710 and 6906 classes: 256 row blocks in one chunk 698 and
+    // 248 (719 and 255 with the other step), 48 in 4 chunks 123 and 36, 18 in 24 chunks 43 and 22
+    // (44 and 22).  Steps of 149 tiles per row block meet in chunks of 37, 74 or 147 tiles: 48 row
+    // blocks 160, 300 in 8 chunks 1019 where these take 810; one chunk 718 and 248.
+    const unsigned step = nsplit == 1 ? kStartStepOne : kStartStepSeveral;
+    const int rot = (int)(((int64_t)((blockIdx.x * step) & 0xffffu) * ntiles) >> 16);
     const int64_t total = nblk * ntiles;
 
     const int tid = threadIdx.x, lane = tid & 63, i = lane & 31, h = lane >> 5;
