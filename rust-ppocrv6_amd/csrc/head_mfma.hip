@@ -262,27 +262,37 @@ static int vec_ok(const float* a, int64_t k) {
 // Vocabulary chunks of the writer (128-row workgroups, one per CU, so 32 per XCD at once).  The
 // count whose grid fills one round best: a multiple of 8 (every XCD its own chunks of every row
 // block) or 4, 2, 1 (an XCD takes one chunk of every 2nd, 4th, 8th row block).  Where that
-// leaves an XCD barely over half full, several rounds of smaller chunks are faster (logits of
-// the 18710-class head, us): 18 row blocks 54 in 8 chunks, 44 in 24; 33 blocks 104 in 4, 95 in
-// 24; fuller ones are not: 23 blocks 55 in 8, 64 in 24; 47 blocks 124 in 4, 144; 94 blocks 244 in
-// 2, 265 in 8; 130 blocks 362 in 1, 372 in 8; 240 blocks 643 in 1, 649 in 8.  (Doubling the count
-// until 192 workgroups, as before, put 18 blocks in 16 chunks: 288 workgroups, two rounds, 60
-// us; 33 in 8: 120; 94 in 4: 283; 130 in 2: 492, its second round 4 workgroups.)
+// leaves an XCD barely over half full, several rounds of 24 smaller chunks are faster if the
+// chunks are of 8 tiles or more (logits, us): 18710 classes, 18 row blocks 54 in 8 chunks, 44 in
+// 24; 33 blocks 104 in 4, 95 in 24; 6906 classes, 18 blocks 23.9 in 8, 22.8 in 24; 65 blocks 65 in
+// 2, 62 in 24.  Smaller chunks are not (4001 classes, 18 blocks 20 in 8, 21 in 24; 65 blocks 47 in 2,
+// 57 in 24; 500 classes, 33 blocks 12 in 4, 21 in 24), nor where the XCD is fuller (18710 classes):
+// 23 blocks 55 in 8, 64 in 24; 47 blocks 124 in 4, 144; 94 blocks 244 in 2, 265 in 8; 130 blocks 362
+// in 1, 372 in 8.  (Doubling the count until 192 workgroups put 18 blocks in 16 chunks: 288
+// workgroups, two rounds, 60 us; 33 in 8: 120; 94 in 4: 283; 130 in 2: 492, its second round 4
+// workgroups.)
 constexpr int kMaxWriterChunks = 128;
-static int rows_nsplit(int64_t mblocks) {
+static int rows_nsplit(int64_t mblocks, int tiles) {
     constexpr int64_t kSlots = 32;  // workgroups of an XCD at once
-    if (mblocks <= kSlots) {
-        const int64_t ns = std::min<int64_t>(8 * (kSlots / mblocks), kMaxWriterChunks);
-        // up to 21 row blocks, two rounds of 24 chunks
-        return ns == 8 && 3 * mblocks <= 2 * kSlots ? 24 : (int)ns;
-    }
-    if (mblocks > 8 * kSlots) {  // more than a round in one chunk: 8 unless its last round is well filled
-        const int64_t last = (mblocks + 7) / 8 % kSlots;
-        return last == 0 || last > 18 ? 1 : 8;
+    if (mblocks > 8 * kSlots) {
+        // More than a round in one chunk: 8 where a last round of few workgroups (it takes (12 +
+        // last / 4) / 32 of a whole one's time: their stores share the bandwidth) costs more than
+        // smaller chunks, in which a workgroup's start is about 6 of its tiles' time.  Us in 1 and
+        // 8 chunks, 18710 classes: 300 blocks 997 and 810, 400 1081 and 1072, 1920 5195 and 5187;
+        // 6906 classes: 300 blocks 344 and 320, 360 356 and 379, 600 592 and 622, 800 817 and
+        // 838; 2049 classes: 300 blocks 111 and 112, 600 201 and 261.
+        const int64_t per_xcd = (mblocks + 7) / 8, last = per_xcd % kSlots;
+        if (last == 0 || last > 18) return 1;
+        const double one = (double)(per_xcd - last) + 12.0 + 0.25 * (double)last;
+        const int tpc = (tiles + 7) / 8;
+        return 0.92 * (double)per_xcd * (tpc + 6) / tpc < one ? 8 : 1;
     }
     int ns = 4;
-    while (ns > 1 && (mblocks * ns + 7) / 8 > kSlots) ns /= 2;
-    return ns > 1 && (mblocks * ns + 7) / 8 <= 18 ? 24 : ns;
+    if (mblocks <= kSlots) ns = (int)std::min<int64_t>(8 * (kSlots / mblocks), kMaxWriterChunks);
+    else
+        while (ns > 1 && (mblocks * ns + 7) / 8 > kSlots) ns /= 2;
+    const bool half = mblocks <= kSlots ? ns == 8 && 3 * mblocks <= 2 * kSlots : ns > 1 && (mblocks * ns + 7) / 8 <= 18;
+    return half && tiles >= 24 * 8 ? 24 : ns;
 }
 
 // Row-block slots of a rescue pass: its grid is sized before the number of guarded rows
@@ -326,7 +336,7 @@ static int launch_rows(int cfg, int epi, const TileGeom& tg, const uint8_t* rec,
     constexpr int ROWS = 32 * kWriterWaves;
     const int64_t mblocks = (m + ROWS - 1) / ROWS;
     if (mblocks > (1 << 24)) return fail(PPOCR_ERR_INVALID_ARG, "MatMulQuantizedB: m too large");
-    const int nsplit = rows_nsplit(mblocks);
+    const int nsplit = rows_nsplit(mblocks, tg.tiles);
     const int tpc = (tg.tiles + nsplit - 1) / nsplit;
     const int64_t grid = grid_blocks((int)mblocks, nsplit, false);
     if (grid > 0x7fffffff) return fail(PPOCR_ERR_INVALID_ARG, "MatMulQuantizedB: m too large");

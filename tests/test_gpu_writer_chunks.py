@@ -51,3 +51,19 @@ def test_writer_rows_and_chunks(orc, rh, m, n):
     assert np.all(np.abs(got[:m * n].reshape(m, n) - pr) <= 2e-4 * scale * pr + 1e-30)
     for d in (da, dout, dws):
         d.free()
+
+
+# 24 chunks in several rounds, 2 chunks, 8 chunks of more than a round of one
+@pytest.mark.parametrize("m,n", [(2305, 6177), (8321, 2049), (33025, 3400)])
+def test_writer_rows_sampled_from_larger_batches(orc, rh, m, n):
+    """Rows from every part of the batch, among them the last row block's, in every class."""
+    rng = np.random.default_rng(m + n)
+    q, s, bias = _head(orc, rng, n, 120)
+    a = rng.standard_normal((m, 120)).astype(np.float32)
+    print(f"writer sampled m={m} n={n}", flush=True)
+    head = rh.RecHead(qw=rh.QuantizedWeight(q, s), bias=bias)
+    rows = np.unique(np.concatenate([rng.choice(m, 300, replace=False), np.arange(m - 130, m)]))
+    got = head.logits(a, 2)[rows]
+    head.close()
+    scale = np.maximum(1.0, np.abs(a[rows]).max(axis=1) / 4.0)[:, None]
+    assert np.all(np.abs(got - f64_logits_q(a[rows], q, s, bias)) <= 1e-4 * scale)
