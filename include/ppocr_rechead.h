@@ -325,6 +325,9 @@ size_t ppocr_rn_workspace_bytes(const ppocr_rn_t* h, int64_t m);
  * by d_line_off[0..lines] (read on the device, clamped into [0, m]; attention never mixes
  * tokens of different lines).  Rows of [0, m) that no line covers (offsets that leave gaps
  * or end before m) have no attention output, and their rows of out are undefined.
+ * d_out may lie over d_x, and over a channels-first d_shortcut, in any way (both are read
+ * whole before the rows that replace them are written); over a d_shortcut of token rows only
+ * as the same buffer.
  * d_workspace: ppocr_rn_workspace_bytes(h, m) bytes, 16-byte aligned, or NULL
  * (stream-ordered scratch). */
 int ppocr_rn_forward_dev(const ppocr_rn_t* h, const float* d_x, const float* d_shortcut, int64_t m,

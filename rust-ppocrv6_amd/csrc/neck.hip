@@ -1311,6 +1311,14 @@ int NeckMark::operator()(const char* name) const {
     return PPOCR_OK;
 }
 
+int launch_cf_rows(const float* src, int64_t m, const int64_t* line_off, int64_t lines, int64_t line_len, float* dst,
+                   hipStream_t st) {
+    const dim3 grid((unsigned)((m + 31) / 32), (unsigned)((kNeckDim + 31) / 32));
+    neck_cf_rows_kernel<<<grid, 256, 0, st>>>(src, m, kNeckDim, line_off, lines, line_len, dst);
+    PPOCR_HIP(hipGetLastError());
+    return PPOCR_OK;
+}
+
 int launch_neck(const NeckDev& nk, const float* x_in, const float* shortcut_in, int64_t m, const int64_t* line_off,
                 int64_t lines, int64_t line_len, int layout, float* out, float* ws, hipStream_t st, NeckMarks* marks) {
     const NeckMark mark{marks, st};
@@ -1336,10 +1344,8 @@ int launch_neck(const NeckDev& nk, const float* x_in, const float* shortcut_in, 
     float* hid = att + m * kNeckAttPad;  // [m][H]
     const float* scr = shortcut_in;
     if (layout == PPOCR_NECK_CHANNELS_FIRST) {
-        const dim3 grid((unsigned)((m + 31) / 32), (unsigned)((D + 31) / 32));
-        neck_cf_rows_kernel<<<grid, 256, 0, st>>>(x_in, m, D, line_off, lines, line_len, x);
-        neck_cf_rows_kernel<<<grid, 256, 0, st>>>(shortcut_in, m, D, line_off, lines, line_len, sc);
-        PPOCR_HIP(hipGetLastError());
+        if (int e = launch_cf_rows(x_in, m, line_off, lines, line_len, x, st)) return e;
+        if (int e = launch_cf_rows(shortcut_in, m, line_off, lines, line_len, sc, st)) return e;
         if (int e = mark("channels_first_to_rows")) return e;
         scr = sc;
     }

@@ -98,13 +98,16 @@ struct NeckMark {
 int launch_neck(const NeckDev& nk, const float* x_in, const float* shortcut_in, int64_t m, const int64_t* line_off,
                 int64_t lines, int64_t line_len, int layout, float* out, float* ws, hipStream_t st,
                 NeckMarks* marks = nullptr);
-// The same on fp16 halves (nk.f16) in one launch per block and one before the first, for at most
-// kNeckFusedRows rows (arguments checked by launch_neck); cf: channels-first input and shortcut.
+// Channels-first rows (as launch_neck's input) to token rows [m][D].
+int launch_cf_rows(const float* src, int64_t m, const int64_t* line_off, int64_t lines, int64_t line_len, float* dst,
+                   hipStream_t st);
 // Fills qkv_h, proj_h, mlp_h and qkv_f .. fc2_f of a block (kNeckPlaneHalves each, in that order)
 // from its uploaded weights and exponents.
 constexpr int kNeckPlaneHalves[7] = {2 * kNeckQkvPad * 128, 2 * kNeckDim * 128, 8 * 16384,
                                      24 * 4 * 1024, 8 * 4 * 1024, 16 * 4 * 1024, 8 * 8 * 1024};
 int launch_neck_planes(const NeckBlockDev& k, hipStream_t st);
+// launch_neck on fp16 halves (nk.f16) in one launch per block and one before the first, for at most
+// kNeckFusedRows rows (arguments checked by launch_neck); cf: channels-first input and shortcut.
 constexpr int64_t kNeckFusedRows = 64 * 256;
 int launch_neck_fused(const NeckDev& nk, const float* x_in, const float* shortcut, int64_t m, const int64_t* line_off,
                       int64_t lines, int64_t line_len, bool cf, float* out, float* ws, hipStream_t st,

@@ -386,9 +386,9 @@ struct Vectors {
     }
 };
 
-// Before the first block: the rows' line table to tab, x (CF: transposed, also to xout) through
-// LN1 and qkv.  Rows whose pointer is not 16-byte aligned are read value by value and also
-// written to xout.
+// Before the first block: the rows' line table to tab, x (CF: transposed) through LN1 and qkv,
+// and its rows to xout where the first block cannot read them where they are (xout not null).
+// Rows whose pointer is not 16-byte aligned are read value by value.
 template <int R, bool CF>
 __global__ __launch_bounds__(kThreads, 2) void neck_qkv_kernel(NeckBlockDev k, float scale, const float* __restrict__ x, int64_t m,
                                                                const int64_t* __restrict__ line_off, int64_t lines,
@@ -433,7 +433,7 @@ __global__ __launch_bounds__(kThreads, 2) void neck_qkv_kernel(NeckBlockDev k, f
         t.store(l.xs, tid);
         __syncthreads();
     }
-    if (CF || !aligned) {
+    if (xout) {
 #pragma unroll
         for (int j = 0; j < U; ++j) {
             const int col = unit_col<R>(part, j);
@@ -812,6 +812,12 @@ __global__ __launch_bounds__(256) void neck_mlp_tiles_kernel(const float* __rest
     }
 }
 
+// Whether two buffers of m rows share memory.
+bool overlap(const float* a, const float* b, int64_t m) {
+    const uintptr_t x = reinterpret_cast<uintptr_t>(a), y = reinterpret_cast<uintptr_t>(b), n = (uintptr_t)m * D * sizeof(float);
+    return x < y + n && y < x + n;
+}
+
 template <int R>
 int go(const NeckDev& nk, const float* x_in, const float* shortcut, int64_t m, const int64_t* line_off, int64_t lines,
        int64_t line_len, bool cf, float* out, float* ws, hipStream_t st, const NeckMark& mark) {
@@ -820,14 +826,25 @@ int go(const NeckDev& nk, const float* x_in, const float* shortcut, int64_t m, c
     uint8_t* qkv[2] = {reinterpret_cast<uint8_t*>(ws + m * D), reinterpret_cast<uint8_t*>(ws + m * (D + kNeckQkvPad))};
     int2* tab = reinterpret_cast<int2*>(ws + m * (D + 2 * kNeckQkvPad));
     static_assert(D + 2 * kNeckQkvPad + 2 <= kNeckWsFloatsPerRow, "x, two qkv buffers and the line table in the workspace");
+    // the residual of the first block: the input rows when they can be read as they are (row by
+    // row while out is written, if the first block is the last)
+    const bool keep = cf || (reinterpret_cast<uintptr_t>(x_in) & 15) || (nk.blocks == 1 && x_in != out && overlap(x_in, out, m));
     (cf ? neck_qkv_kernel<R, true> : neck_qkv_kernel<R, false>)<<<grid, kThreads, sizeof(Lds<R>), st>>>(
-        nk.block[0], nk.scale, x_in, m, line_off, lines, line_len, tab, x, qkv[0]);
+        nk.block[0], nk.scale, x_in, m, line_off, lines, line_len, tab, keep ? x : nullptr, qkv[0]);
     PPOCR_HIP(hipGetLastError());
     if (int e = mark("ln1_qkv")) return e;
-    // the residual of the first block: the input rows when they can be read as they are
-    const float* xr = cf || (reinterpret_cast<uintptr_t>(x_in) & 15) ? x : x_in;
+    const float* xr = keep ? x : x_in;
     for (int b = 0; b < nk.blocks; ++b, xr = x) {
         const bool last = b + 1 == nk.blocks;
+        if (last && cf && overlap(shortcut, out, m)) {
+            // a workgroup's rows of out lie over other workgroups' part of the shortcut: its rows
+            // first, into the qkv buffer that no kernel reads any more
+            float* rows = reinterpret_cast<float*>(qkv[(b + 1) & 1]);
+            if (int e = launch_cf_rows(shortcut, m, line_off, lines, line_len, rows, st)) return e;
+            if (int e = mark("channels_first_to_rows")) return e;
+            shortcut = rows;
+            cf = false;
+        }
         auto* kern = !last ? neck_block_kernel<R, false, false>
                      : cf  ? neck_block_kernel<R, true, true>
                            : neck_block_kernel<R, true, false>;
