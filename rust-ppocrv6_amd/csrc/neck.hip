@@ -25,6 +25,7 @@
 
 #include "kernels.hpp"
 #include "neck.hpp"
+#include "neck_device.hpp"
 
 namespace ppocr {
 
@@ -517,7 +518,6 @@ constexpr int kMlpConstChunks = 256;
 static_assert(kMlpW1 == 0 && kMlpRows * kNeckDim * 4 <= kMlpRing1 * kMlpPart, "the rows of x fit the fc1 ring");
 constexpr size_t mlp16_lds_bytes() { return (size_t)kMlpConst + kMlpConstChunks * 16; }
 
-__device__ __forceinline__ float swish_fast(float z) { return z * __builtin_amdgcn_rcpf(1.0f + __expf(-z)); }
 
 // FINAL (the last block): the rows are then taken through the final LayerNorm and the
 // shortcut Add (neck_final_kernel's arithmetic) before the store, into fin_out.
@@ -839,20 +839,6 @@ constexpr int kVtStride = kAttnKeys + 4;
 
 __device__ __forceinline__ int perm_dim(int d) { return 4 * (d & 3) + (d >> 2); }
 
-// max(a, b) as one v_max_f32 (fmaxf on values the compiler cannot prove canonical, MFMA
-// results and shuffles, costs a v_max_f32 x, x, x per operand first).  Operands here are
-// scores, never NaN unless the inputs are.
-__device__ __forceinline__ float max_f32(float a, float b) {
-    float r;
-    asm("v_max_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
-    return r;
-}
-__device__ __forceinline__ float max3_f32(float a, float b, float c) {
-    float r;
-    asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
-    return r;
-}
-
 template <int HD>
 __global__ __launch_bounds__(256) void neck_attn_kernel(const float* __restrict__ qkv, int64_t m,
                                                         const int64_t* __restrict__ line_off, int64_t lines,
@@ -929,6 +915,8 @@ __global__ __launch_bounds__(256) void neck_attn_kernel(const float* __restrict_
                     for (int s = 0; s < 4; ++s) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[s], qf[x][s], acc, 0, 0, 0);
                     sc[t] = acc;
                 }
+#pragma unroll
+                for (int t = 0; t < KT; t += 4) settle_f32(sc[t], sc[t + 1], sc[t + 2], sc[t + 3]);
                 // keys past the line's end score -inf (their p is then exactly 0); the block's
                 // maximum for query q0 + c: this lane's keys, then the lane groups
                 float bm = -INFINITY;
@@ -937,12 +925,12 @@ __global__ __launch_bounds__(256) void neck_attn_kernel(const float* __restrict_
 #pragma unroll
                     for (int jj = 0; jj < 4; ++jj) {
                         sc[t][jj] = (16 * t + 4 * g + jj < rem) ? sc[t][jj] : -INFINITY;
-                        bm = max_f32(bm, sc[t][jj]);
+                        bm = max_settled(bm, sc[t][jj]);
                     }
                 }
-                bm = max_f32(bm, __shfl_xor(bm, 16, 64));
-                bm = max_f32(bm, __shfl_xor(bm, 32, 64));
-                const float nm = max_f32(mx[x], bm);
+                bm = max_settled(bm, __shfl_xor(bm, 16, 64));
+                bm = max_settled(bm, __shfl_xor(bm, 32, 64));
+                const float nm = max_settled(mx[x], bm);
                 if (kb > 0) {
                     // rescale the sums so far (every block of a pass after the first follows one
                     // that set a finite maximum)
@@ -1128,6 +1116,8 @@ __global__ __launch_bounds__(256) void neck_attn16_kernel(const float* __restric
                         acc = __builtin_amdgcn_mfma_f32_16x16x16f16(kh, ql[x], acc, 0, 0, 0);
                         sc[u] = __builtin_amdgcn_mfma_f32_16x16x16f16(kl, qh[x], acc, 0, 0, 0);
                     }
+                    static_assert(KS == 4, "one wait for the sub-block's scores");
+                    settle_f16(sc[0], sc[1], sc[2], sc[3]);
                     // keys past the line's end score -inf (their p is then exactly 0), tested only
                     // in the tiles that reach past it; the sub-block's maximum for query q0 + c:
                     // this lane's keys, then the lane groups
@@ -1141,11 +1131,11 @@ __global__ __launch_bounds__(256) void neck_attn16_kernel(const float* __restric
                             for (int jj = 0; jj < 4; ++jj)
                                 sc[u][jj] = (16 * t + 4 * g + jj < rem) ? sc[u][jj] : -INFINITY;
                         }
-                        bm = max3_f32(max3_f32(bm, sc[u][0], sc[u][1]), sc[u][2], sc[u][3]);
+                        bm = max3_settled(max3_settled(bm, sc[u][0], sc[u][1]), sc[u][2], sc[u][3]);
                     }
-                    bm = max_f32(bm, __shfl_xor(bm, 16, 64));
-                    bm = max_f32(bm, __shfl_xor(bm, 32, 64));
-                    const float nm = max_f32(mx[x], bm);
+                    bm = max_settled(bm, __shfl_xor(bm, 16, 64));
+                    bm = max_settled(bm, __shfl_xor(bm, 32, 64));
+                    const float nm = max_settled(mx[x], bm);
                     if (kb > 0 || sb > 0) {
                         // rescale the sums so far (every sub-block after the pass's first follows
                         // one that set a finite maximum: its first key is inside the line)

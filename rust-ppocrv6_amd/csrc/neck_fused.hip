@@ -31,6 +31,7 @@
 
 #include "kernels.hpp"
 #include "neck.hpp"
+#include "neck_device.hpp"
 
 namespace ppocr {
 
@@ -73,30 +74,15 @@ __device__ __forceinline__ f32x4 mfma32(f16x8 a, f16x8 b, f32x4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
 }
 
-// max as one v_max_f32 (fmaxf on values the compiler cannot prove canonical costs a
-// v_max_f32 x, x, x per operand first)
-__device__ __forceinline__ float vmax(float a, float b) {
-    float r;
-    asm("v_max_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
-    return r;
-}
-__device__ __forceinline__ float vmax3(float a, float b, float c) {
-    float r;
-    asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
-    return r;
-}
-
 // The maximum over the lanes c, c + 16, c + 32, c + 48, in each of them: the swaps exchange
 // odd with even rows of 16 lanes, then the halves, in the vector ALU (no trip through LDS).
 __device__ __forceinline__ float max_over_groups(float x) {
     const unsigned u = __float_as_uint(x);
     const auto a = __builtin_amdgcn_permlane16_swap(u, u, false, false);
-    const unsigned y = __float_as_uint(vmax(__uint_as_float(a[0]), __uint_as_float(a[1])));
+    const unsigned y = __float_as_uint(max_f32(__uint_as_float(a[0]), __uint_as_float(a[1])));
     const auto b = __builtin_amdgcn_permlane32_swap(y, y, false, false);
-    return vmax(__uint_as_float(b[0]), __uint_as_float(b[1]));
+    return max_f32(__uint_as_float(b[0]), __uint_as_float(b[1]));
 }
-
-__device__ __forceinline__ float swish(float z) { return z * __builtin_amdgcn_rcpf(1.0f + __expf(-z)); }
 
 template <int R>
 struct Lds {
@@ -547,10 +533,10 @@ __device__ __forceinline__ void attention(Lds<R>& l, const NeckBlockDev& k, cons
 #pragma unroll
                         for (int j = 0; j < 4; ++j) sc[u][j] = (16 * u + 4 * g + j < rem) ? sc[u][j] : -INFINITY;
                     }
-                    bm = vmax3(vmax3(bm, sc[u][0], sc[u][1]), sc[u][2], sc[u][3]);
+                    bm = max3_f32(max3_f32(bm, sc[u][0], sc[u][1]), sc[u][2], sc[u][3]);
                 }
                 bm = max_over_groups(bm);
-                const float nm = vmax(mx[rt], bm);
+                const float nm = max_f32(mx[rt], bm);
                 // every step has a key inside the line, so nm is finite
                 if (kb > 0) oa[rt] = oa[rt] * __builtin_amdgcn_exp2f((mx[rt] - nm) * ec);
                 mx[rt] = nm;
@@ -665,7 +651,7 @@ __global__ __launch_bounds__(kThreads, 2) void neck_block_kernel(
                 u32x2 hi, lo;
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
-                    z[e] = swish(acc[t][rt][e] * s + b1[e]) * sh;
+                    z[e] = swish_fast(acc[t][rt][e] * s + b1[e]) * sh;
                     z[e] = unit < H ? z[e] : 0.0f;
                 }
                 split4(z, hi, lo);

@@ -26,7 +26,7 @@ const SOURCES: &[&str] = &[
     "model_graph.cpp",
 ];
 const HEADERS: &[&str] =
-    &["common.hpp", "kernels.hpp", "neck.hpp", "head_mfma.hpp", "safetensors.hpp", "json.hpp", "model_graph.hpp"];
+    &["common.hpp", "kernels.hpp", "neck.hpp", "neck_device.hpp", "head_mfma.hpp", "safetensors.hpp", "json.hpp", "model_graph.hpp"];
 const FLAGS: &[&str] = &[
     "--offload-arch=gfx950",
     "-O3",
