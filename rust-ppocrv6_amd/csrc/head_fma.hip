@@ -97,22 +97,51 @@ __global__ __launch_bounds__(256, EPI == EPI_STATS || GATHER ? 2 : 3) void head_
         // another one of the batch (its results are never stored, and each result depends on its
         // own row and class alone).
         const int kq = 4 * (tid & 3), kq_last = (nk - 1) * KC + kq < k ? kq : 0;
+        // Otherwise value by value: k = tid % 16 of rows and classes tid / 16 + 16 it (channels
+        // first: row tid % 128, k = tid / 128 + 2 it, so neighbouring threads take neighbouring
+        // steps), into the same registers and a step later into the LDS buffer.  (Loaded and
+        // stored in one step, so that every step waited for memory: the statistics of 512 rows
+        // of an FP32 head of 18710 x 121 131 us, 82 so, 7680 rows 928 and 720; the vector ALU's
+        // kernel, more waves at once, 106 and 1125.)
+        const int64_t any = m0 < m ? m0 : 0;
         int64_t arow[2];
-        // channels first: where this thread's row (tid % 128) starts, at k = 0
-        int64_t cf_row = -1;
+        int64_t cf_row = 0;  // channels first: where this thread's row starts, at k = 0
         unsigned woff[2] = {0, 0};
         if constexpr (VEC) {
 #pragma unroll
             for (int it = 0; it < 2; ++it) {
                 const int64_t row = s_row[(tid >> 2) + 64 * it];
-                arow[it] = (row >= 0 ? row : m0 < m ? m0 : 0) * k;
+                arow[it] = (row >= 0 ? row : any) * k;
             }
         } else if (line_len > 0) {
-            const int64_t row = s_row[tid & (BM - 1)];
-            if (row >= 0) cf_row = row / line_len * k * line_len + row % line_len;
+            const int64_t row = s_row[tid & (BM - 1)], r = row >= 0 ? row : any;
+            cf_row = r / line_len * k * line_len + r % line_len;
         }
         f32x4 ca[2], cw[2];
         auto load = [&](int n0, int x) {
+            if constexpr (!VEC) {
+                int t = tid;
+                asm volatile("" : "+v"(t));  // addresses from here on: kept over the loop they would spill
+                const int kl = k - 1, kk = min(x * KC + (t & 15), kl);
+                if (line_len > 0) {
+                    const float* p = a + cf_row;
+#pragma unroll
+                    for (int it = 0; it < 8; ++it) ca[it >> 2][it & 3] = p[min(x * KC + (t >> 7) + 2 * it, kl) * line_len];
+                } else {
+#pragma unroll
+                    for (int it = 0; it < 8; ++it) {
+                        const int64_t row = s_row[(t >> 4) + 16 * it];
+                        ca[it >> 2][it & 3] = a[(row >= 0 ? row : any) * k + kk];
+                    }
+                }
+#pragma unroll
+                for (int it = 0; it < 8; ++it) {
+                    const int64_t e = (int64_t)min(n0 + (t >> 4) + 16 * it, n - 1) * k + kk;
+                    if constexpr (Q) cw[it >> 2][it & 3] = __int_as_float((int)q[e]);
+                    else cw[it >> 2][it & 3] = w[e];
+                }
+                return;
+            }
             if (x == 0) {
 #pragma unroll
                 for (int it = 0; it < 2; ++it) woff[it] = (unsigned)min((tid >> 2) + 64 * it, n - 1 - n0) * (unsigned)k;
@@ -128,6 +157,21 @@ __global__ __launch_bounds__(256, EPI == EPI_STATS || GATHER ? 2 : 3) void head_
             }
         };
         auto put = [&](int buf, int x) {
+            if constexpr (!VEC) {
+                int t = tid;
+                asm volatile("" : "+v"(t));
+                float* as = lf + (size_t)buf * (BM + BN) * LST;
+                const int o = (t >> 4) * LST + (t & 15), oc = (t & (BM - 1)) * LST + (t >> 7);
+                const bool in = x * KC + (t & 15) < k;  // past k: zeros
+#pragma unroll
+                for (int it = 0; it < 8; ++it) {
+                    const float v = ca[it >> 2][it & 3], u = cw[it >> 2][it & 3];
+                    if (line_len > 0) as[oc + 2 * it] = x * KC + (t >> 7) + 2 * it < k ? v : 0.0f;
+                    else as[o + 16 * it * LST] = in ? v : 0.0f;
+                    as[BM * LST + o + 16 * it * LST] = in ? (Q ? (float)__float_as_int(u) : u) : 0.0f;
+                }
+                return;
+            }
             float* as = lf + (size_t)buf * (BM + BN) * LST + (tid >> 2) * LST + kq;
             if constexpr (Q) {
 #pragma unroll
@@ -143,33 +187,6 @@ __global__ __launch_bounds__(256, EPI == EPI_STATS || GATHER ? 2 : 3) void head_
             for (int it = 0; it < 2; ++it) {
                 *reinterpret_cast<f32x4*>(as + 64 * it * LST) = ca[it];
                 *reinterpret_cast<f32x4*>(as + (BM + 64 * it) * LST) = cw[it];
-            }
-        };
-        // Otherwise value by value straight into the LDS buffer: k = tid % 16 of rows and classes
-        // tid / 16 + 16 it (channels first: row tid % 128, k = tid / 128 + 2 it, so neighbouring
-        // threads take neighbouring steps).  Past the rows, classes or k: zeros.
-        auto stage = [&](int n0, int x, int buf) {
-            float* as = lf + (size_t)buf * (BM + BN) * LST;
-            float* ws = as + BM * LST;
-#pragma unroll 4
-            for (int it = 0; it < BM * KC / 256; ++it) {
-                if (line_len > 0) {
-                    const int kk = (tid >> 7) + 2 * it;
-                    as[(tid & (BM - 1)) * LST + kk] =
-                        cf_row >= 0 && x * KC + kk < k ? a[cf_row + (x * KC + kk) * line_len] : 0.0f;
-                } else {
-                    const int r = (tid >> 4) + 16 * it, kk = x * KC + (tid & 15);
-                    const int64_t row = s_row[r];
-                    as[r * LST + (tid & 15)] = row >= 0 && kk < k ? a[row * k + kk] : 0.0f;
-                }
-                const int c = (tid >> 4) + 16 * it, kk = x * KC + (tid & 15);
-                float v = 0.0f;
-                if (n0 + c < c1 && kk < k) {
-                    const int64_t e = (int64_t)(n0 + c) * k + kk;
-                    if constexpr (Q) v = (float)q[e];
-                    else v = w[e];
-                }
-                ws[c * LST + (tid & 15)] = v;
             }
         };
         // the constants of the tile from n0 (zeros past the chunk): loaded by the first 128
@@ -226,13 +243,9 @@ __global__ __launch_bounds__(256, EPI == EPI_STATS || GATHER ? 2 : 3) void head_
                 for (int t = 0; t < 4; ++t) acc[t] = product(f, e, t, acc[t]);
         };
         Step s0{c0, 0}, s1 = next(s0);
-        if constexpr (VEC) {
-            load(c0, 0);
-            put(0, 0);
-            if (s1.n0 < c1) load(s1.n0, s1.x);
-        } else {
-            stage(c0, 0, 0);
-        }
+        load(c0, 0);
+        put(0, 0);
+        if (s1.n0 < c1) load(s1.n0, s1.x);
         load_const(c0);
         put_const(0);
         if (nk == 1 && s1.n0 < c1) load_const(s1.n0);
@@ -244,8 +257,7 @@ __global__ __launch_bounds__(256, EPI == EPI_STATS || GATHER ? 2 : 3) void head_
             for (int x = 0; x < nk; ++x) {
                 const bool more = s1.n0 < c1;
                 if (more) {
-                    if constexpr (VEC) put(buf ^ 1, s1.x);
-                    else stage(s1.n0, s1.x, buf ^ 1);
+                    put(buf ^ 1, s1.x);
                     // the constants of four tiles: a slower wave may still read the last tile's
                     if (s1.x == 0) put_const((par + 1) & 3);
                 }
@@ -263,7 +275,7 @@ __global__ __launch_bounds__(256, EPI == EPI_STATS || GATHER ? 2 : 3) void head_
                 __syncthreads();
                 const Step s2 = next(s1);
                 if (s2.n0 < c1) {
-                    if constexpr (VEC) load(s2.n0, s2.x);
+                    load(s2.n0, s2.x);
                     if (s2.x == 0) load_const(s2.n0);
                 }
                 buf ^= 1;
