@@ -47,3 +47,47 @@ def test_fp32_tiles(orc, rh, m, n, k, fp32):
     rel = 2 * bound.max() + 4e-6
     assert np.all(np.abs(p - pr) <= rel * pr + 1e-30)
     assert np.all(np.abs(d["maxprob"] - pr.max(axis=1)) <= rel * pr.max(axis=1))
+
+
+def _chunks(head, m):
+    """Vocabulary chunks of the statistics pass, from the partials' share of the workspace."""
+    def up(x):
+        return (x + 255) // 256 * 256
+    return (head.workspace_bytes(m, 0) - 256 - 3 * up(4 * m) - up((m + 127) // 128)) // (12 * m)
+
+
+@pytest.mark.parametrize("fp32", [False, True])
+@pytest.mark.parametrize("k", [4, 15, 16, 20, 32, 121])
+@pytest.mark.parametrize("n", [385, 1025])
+def test_statistics_over_several_tiles(orc, rh, n, k, fp32):
+    """So many row blocks that a workgroup walks several tiles of classes: two, or five (one
+    more than the buffers of scale and bias), with one or more chunks of k each, 4 values of k
+    at a time or one by one, rows or channels first.  Sampled rows against 64 bits; the two
+    layouts give the same bits."""
+    rng = np.random.default_rng(n + k + fp32)
+    lines, steps = 550, 120
+    m = lines * steps
+    w = (rng.standard_normal((n, k)) * 0.3).astype(np.float32)
+    bias = (rng.standard_normal(n) * 0.5).astype(np.float32)
+    if fp32:
+        head, wd = rh.RecHead(w_t=w, bias=bias), w.astype(np.float64)
+    else:
+        q, s = orc.pack_int8(w)
+        head = rh.RecHead(qw=rh.QuantizedWeight(q, s), bias=bias)
+        wd = q.astype(np.float64) * s.astype(np.float64)[:, None]
+    tiles = (n + 127) // 128
+    per_chunk = -(-tiles // _chunks(head, m))
+    print(f"fp32 statistics n={n} k={k} fp32={fp32}: {per_chunk} tiles a chunk", flush=True)
+    assert per_chunk >= (2 if n == 385 else 5)
+    a = rng.standard_normal((m, k)).astype(np.float32)
+    off = (np.arange(lines + 1) * steps).astype(np.int64)
+    got = head.decode(a, off, 0)
+    cf = head.decode_nct(np.ascontiguousarray(a.reshape(lines, steps, k).transpose(0, 2, 1)), 0)
+    head.close()
+    assert np.array_equal(cf["idx"], got["idx"]) and np.array_equal(cf["maxprob"], got["maxprob"])
+    rows = np.unique(np.concatenate([rng.choice(m, 400, replace=False), np.arange(m - 90, m)]))
+    ref = a[rows].astype(np.float64) @ wd.T + bias.astype(np.float64)
+    bound = (k + 2) * 2.0**-24 * (np.abs(a[rows]).astype(np.float64) @ np.abs(wd).T + np.abs(bias)).max()
+    check_argmax(got["idx"][rows], ref.argmax(axis=1), top2_gap(ref), tol=2 * bound)
+    p = 1.0 / np.exp(ref - ref.max(axis=1, keepdims=True)).sum(axis=1)
+    assert np.all(np.abs(got["maxprob"][rows] - p) <= (2 * bound + 4e-6) * p)
