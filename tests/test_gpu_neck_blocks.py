@@ -80,3 +80,39 @@ def test_unaligned_input_rows(rh):
     for d in (dx, ds, doff, dout, dws):
         d.free()
     neck.close()
+
+
+@pytest.mark.parametrize("lengths", [[33, 90], [120] * 40, [240] * 40], ids=["tiles of 16", "tiles of 32", "tiles of 64"])
+@pytest.mark.parametrize("cf", [False, True], ids=["rows", "channels first"])
+def test_unaligned_rows(rh, cf, lengths):
+    """Each of x, the shortcut and the output, and all of them, 4 bytes off a 16-byte boundary:
+    the same bits as the aligned ones, and nothing written around the output."""
+    from ppocr_rechead.hip import DeviceArray, synchronize
+    w = neck_weights(seed=53)
+    neck = _make(rh, w)
+    x, sc, off = _inputs(lengths, seed=21)
+    m = int(off[-1])
+    want = neck.forward(x, sc, off)
+    if cf:
+        x, sc = rows_to_cf(x, off), rows_to_cf(sc, off)
+    doff = DeviceArray.from_numpy(off)
+    wsb = neck.workspace_bytes(m)
+    dws = DeviceArray((wsb,), np.uint8)
+    for mask in (1, 2, 4, 7):
+        at = [1 if mask >> b & 1 else 0 for b in range(3)]
+        ds = [DeviceArray.from_numpy(np.concatenate([np.zeros(o), v.reshape(-1), np.zeros(4)]).astype(np.float32))
+              for o, v in zip(at, (x, sc))]
+        dout = DeviceArray.from_numpy(np.full(m * DIM + 5, 7.0, np.float32))
+        ptr = [ctypes.c_void_p(d.p.value + 4 * o) for d, o in zip((*ds, dout), at)]
+        rh._check(rh._lib.lib().ppocr_rn_forward_dev(neck.handle, ptr[0], ptr[1], m, doff.p, len(lengths),
+                                                     rh.NECK_CHANNELS_FIRST if cf else rh.NECK_ROWS, ptr[2], dws.p, wsb,
+                                                     None))
+        synchronize()
+        got = dout.numpy()
+        assert np.array_equal(got[at[2]:at[2] + m * DIM].reshape(m, DIM), want), mask
+        assert np.all(got[:at[2]] == 7.0) and np.all(got[at[2] + m * DIM:] == 7.0), mask
+        for d in (*ds, dout):
+            d.free()
+    for d in (doff, dws):
+        d.free()
+    neck.close()
