@@ -100,16 +100,15 @@ struct DeviceGuard {
 // Device memory of the host-pointer entry points.  Each call takes an arena (one device
 // allocation, a pinned host staging buffer and a stream of its own) from a pool, lays its
 // inputs, outputs and workspace out in it, and gives it back, so a call costs its copies
-// and kernels rather than allocations.  Inputs and outputs of up to kStageBytes move as
-// one copy each way through the pinned buffer; larger ones are copied directly.  Calls
-// running at the same time take different arenas.  The staged inputs go to the device in pieces,
-// by a kernel that reads the pinned buffer, so a piece crosses PCIe while the next one is being
-// copied into the buffer and the call's kernels follow on the same queue; decoded results of
-// up to kDirectBytes are written by the kernels into the pinned buffer themselves.  (An A4 page,
-// 2245 rows from host arrays: 107 us with one asynchronous copy each way, 96 so.)
-// Arenas above kArenaKeepBytes are freed
-// after the call instead of kept (the logits of a large batch need gigabytes once).  The
-// pool lives until the process ends.
+// and kernels rather than allocations.  Calls running at the same time take different arenas.
+// Inputs of up to kStageBytes go through the pinned buffer in pieces: a kernel that reads the
+// buffer takes a piece across PCIe while the next one is being copied into it, and the call's
+// kernels follow on the same queue.  Decoded results of up to kDirectBytes are written by the
+// kernels into the pinned buffer themselves, other outputs of up to kStageBytes come back through
+// it in one copy.  Larger inputs and outputs are copied directly.  (An A4 page, 2245 rows from
+// host arrays, the call from C: 107 us with one asynchronous copy each way, 96 so.)  Arenas above
+// kArenaKeepBytes are freed after the call instead of kept (the logits of a large batch need
+// gigabytes once).  The pool lives until the process ends.
 constexpr size_t kArenaKeepBytes = 256u << 20;
 constexpr size_t kStageBytes = 4u << 20;
 constexpr size_t kDirectBytes = 256u << 10;  // after the stage, in the same pinned buffer

@@ -7,8 +7,9 @@
 // from registers on this chip, against 78 for the vector ALU's v_fma_f32 without packing).  A
 // workgroup's tile is 128 rows x 128 classes: wave w owns rows 32 w .. + 31 and all 128 classes
 // (four 32x32 accumulators), so a softmax statistic never crosses waves.  k passes through LDS
-// in chunks of 16, two buffers (41 KB, so three workgroups per CU: chunks of 32 and two per CU
-// took 377 us where this takes 363); within 8 values of k lane half h holds k = 4 h .. 4 h + 3,
+// in chunks of 16, two buffers (41 KB, so three workgroups per CU for the logits and the
+// probabilities: chunks of 32 and two per CU took 377 us where this takes 363; the statistics
+// and the rescues, with more registers, run two per CU); within 8 values of k lane half h holds k = 4 h .. 4 h + 3,
 // one 16-byte LDS read for four MFMA steps (step e multiplies k = e and k = 4 + e), so a wave
 // reads 5 KB of LDS per 16 MFMAs.
 // Measured, 7680 x 120 x 18710 (an FP32 head's logits, 34.5 GFLOP, 575 MB written): 802 us with

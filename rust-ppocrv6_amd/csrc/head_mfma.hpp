@@ -1155,7 +1155,7 @@ __global__ __launch_bounds__(64 * (kWriterWaves + 1), 1) void rows_w_kernel(
                 // so are classes past n, moved past any end.  A branch per row instead made the
                 // compiler wait for the stores in flight: a batch that is no multiple of 128 rows
                 // waited for its last row block (12000 rows of the 18710-class head in one chunk
-                // took 381 us with its row branches, 326 as 93 whole row blocks, 338 so).  Whole
+                // took 381 us with its row branches, whole row blocks 326; 338 so).  Whole
                 // tiles as well through the buffer took longer: 6144 rows of a 6906-class head 39
                 // us, 36 so.
                 const unsigned o = col < n ? ((unsigned)(4 * h) * (unsigned)n + (unsigned)col) * 4u : 0xFFFFFFFFu;

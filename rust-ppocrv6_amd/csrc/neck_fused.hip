@@ -865,7 +865,11 @@ int launch_neck_fused(const NeckDev& nk, const float* x_in, const float* shortcu
     if (m > kNeckFusedRows) return fail(PPOCR_ERR_INVALID_ARG, "RecNeckHip: too many rows");
     // the smallest tile whose grid is at most a workgroup per CU: fewer rows, a shorter chain.
     // Measured (lines of 128, rows first): 128 rows 30 / 39 / 60 us with tiles of 16 / 32 / 64
-    // rows, 4096: 40 / 45 / 66, 8192: 69 / 51 / 68, 16384: 128 / 89 / 76
+    // rows, 4096: 40 / 45 / 66, 8192: 69 / 51 / 68, 16384: 128 / 89 / 76.  A tile's lines are
+    // taken one after another, so lines of a row or two make a chain of it: 64 lines of one row 70
+    // us, 4096 of one row 77, 8194 of one row 283, 2049 of four 111; the separate kernels, a
+    // workgroup per line and head, take 69, 231, 396 and 162.  One line of 1000 rows 66, of 16384
+    // rows 1415; the separate kernels 461 and 105410
     auto f = m <= 16 * 256 ? go<16> : m <= 32 * 256 ? go<32> : go<64>;
     return f(nk, x_in, shortcut, m, line_off, lines, line_len, cf, out, ws, st, mark);
 }
