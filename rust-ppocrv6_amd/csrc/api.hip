@@ -1011,7 +1011,7 @@ int ppocr_argmax_rows(const float* x, int64_t rows, int64_t cols, int32_t* idx, 
     if ((!x && cols) || !idx || !val) return fail(PPOCR_ERR_INVALID_ARG, "CtcDecode: null pointer");
     const size_t xb = (size_t)(rows * cols) * 4, rb = (size_t)rows * 4;
     HostCall hc;
-    if (int e = hc.begin({xb}, {rb, rb}, 0)) return e;
+    if (int e = hc.begin({xb}, {rb, rb}, 0, true)) return e;
     if (int e = hc.copy_in({x})) return e;
     if (int e = launch_argmax_rows(hc.in<float>(0), rows, cols, hc.out<int32_t>(0), hc.out<float>(1), hc.stream()))
         return e;
@@ -1121,7 +1121,7 @@ int ppocr_ctc_greedy(const int32_t* idx, const float* maxprob, const int64_t* li
     if (steps > 0 && (!idx || !maxprob || !seq)) return fail(PPOCR_ERR_INVALID_ARG, "CtcDecode: null pointer");
     const size_t sb = (size_t)steps * 4, ob = (size_t)(lines + 1) * 8;
     HostCall hc;
-    if (int e = hc.begin({sb, sb, ob}, {sb, (size_t)lines * 8, (size_t)lines * 4}, 0)) return e;
+    if (int e = hc.begin({sb, sb, ob}, {sb, (size_t)lines * 8, (size_t)lines * 4}, 0, true)) return e;
     if (int e = hc.copy_in({idx, maxprob, line_off})) return e;
     if (int e = launch_ctc_greedy(hc.in<int32_t>(0), hc.in<float>(1), hc.in<int64_t>(2), lines, blank,
                                   hc.out<int32_t>(0), hc.out<int64_t>(1), hc.out<float>(2), hc.stream()))

@@ -63,3 +63,28 @@ def test_host_decode_nct_across_the_staging_sizes(rh, orc):
         for d in (dx, di, dm, dq, dl, ds, dw):
             d.free()
     head.close()
+
+
+def test_host_argmax_and_ctc_across_the_pinned_results(rh):
+    """ppocr_argmax_rows and ppocr_ctc_greedy with results around 256 KB, where they leave the
+    pinned buffer."""
+    rng = np.random.default_rng(7)
+    for rows in (1, 32767, 32768, 32769):  # two results of 128 KB
+        x = rng.standard_normal((rows, 5)).astype(np.float32)
+        idx, val = np.zeros(rows, np.int32), np.zeros(rows, np.float32)
+        rh._check(rh._lib.lib().ppocr_argmax_rows(rh._ptr(x), rows, 5, rh._ptr(idx), rh._ptr(val)))
+        assert np.array_equal(idx, x.argmax(axis=1)) and np.array_equal(val, x.max(axis=1)), rows
+    for steps in (1, 64, 65000, 65400, 65536, 65600):  # the tokens, 8 + 4 bytes a line
+        ids = rng.integers(0, 3, steps).astype(np.int32)
+        p = rng.random(steps).astype(np.float32)
+        off = np.array([0, steps // 3, steps], np.int64)
+        seqs, score = rh.CtcDecoder.collapse(ids, p, off)
+        for b in range(2):
+            i = ids[off[b]:off[b + 1]]
+            keep = i != 0
+            keep[1:] &= i[1:] != i[:-1]
+            assert np.array_equal(seqs[b], i[keep]), (steps, b)
+            total = np.float32(0.0)
+            for v in p[off[b]:off[b + 1]][keep]:
+                total += v
+            assert score[b] == (total / np.float32(keep.sum()) if keep.any() else 0.0), (steps, b)
