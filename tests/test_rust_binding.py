@@ -173,7 +173,7 @@ def _added(patch):
                      if l.startswith("+") and not l.startswith("+++"))
 
 
-@pytest.mark.skipif(not os.path.isdir(REF) or not shutil.which("patch"), reason="the reference crate is not here")
+@pytest.mark.skipif(not os.path.isdir(os.path.join(REF, "src")) or not shutil.which("patch"), reason="the reference crate is not here")
 def test_patches_apply_to_the_reference_and_are_current(tmp_path):
     for patch, rel in PATCHES.items():
         dst = tmp_path / rel
