@@ -300,6 +300,15 @@ static int rows_nsplit(int64_t mblocks, int tiles) {
 // rescue costs the launch whatever the grid, and a heavy one (a head with large weight
 // outliers guards many rows) needs the whole GPU.
 constexpr int kRescueSlots = 128;
+// Vocabulary chunks of the writer's rescue: its own count, doubled until the row blocks make 192
+// workgroups of it.  A single round of fewer leaves a rescue of some rows to few workgroups, each
+// walking a long chunk (logits with 2% of the rows guarded, 18710 classes, us, in the writer's
+// chunks and these: 22 row blocks 123 and 93, 80 blocks 459 and 348, 129 blocks 850 and 619; all
+// guarded 125 and 130, 480 and 516, 1253 and 958).
+static int rescue_nsplit(int64_t mblocks, int nsplit) {
+    while (mblocks * nsplit < 192 && nsplit < 64) nsplit *= 2;
+    return nsplit;
+}
 // Workgroups of a statistics rescue: one round of the GPU at the three-term pass's two
 // workgroups per CU.  A larger grid walks no more blocks at once (a full list of 18 blocks
 // in 64 chunks takes three rounds either way) and an empty list still dispatches all of it.
@@ -381,7 +390,9 @@ static int launch_rows(int cfg, int epi, const TileGeom& tg, const uint8_t* rec,
                                  nullptr, 0, *guard, st);
     // rescue: the flagged rows again, three bf16 activation terms, every column
     const int slots = (int)std::min<int64_t>(mblocks, kRescueSlots);
-    const int rgrid = grid_blocks(slots, nsplit, false);
+    x.nsplit = rescue_nsplit(mblocks, nsplit);
+    x.tpc = (tg.tiles + x.nsplit - 1) / x.nsplit;
+    const int rgrid = grid_blocks(slots, x.nsplit, false);
     x.rec = rec_rescue;
     x.mblocks = slots;
     x.lim = none;
